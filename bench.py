@@ -102,12 +102,15 @@ def kernel_symbol(info, cls, precision=0):
         return "eri_" + info[name]["split_kernels"][fam - 3]
     if fam in (5, 6):
         return "eri_" + info[name]["split_kernels_f"][fam - 5]
+    if fam == 7:
+        return "eri_cpl_%s" % name
     return "eri_wpq_%s" % name
 
 
 def list_kernel_symbol(cls):
     import simint
-    return ("eri_lpql_%s" if simint.lib().simint_hip_class_list_kernel(*cls) == 1 else "eri_wpql_%s") % cname(cls)
+    fam = simint.lib().simint_hip_class_list_kernel(*cls)
+    return {1: "eri_lpql_%s", 7: "eri_cpll_%s"}.get(fam, "eri_wpql_%s") % cname(cls)
 
 
 def shares(launches, k):
@@ -462,7 +465,7 @@ def batched_leg(steps, warmup, nquartet=10 ** 6):
                            for ms, g in per[:8]]}
     fam = {}
     for ms, g in per:
-        k = "wpql" if "wpql" in list_kernel_symbol(g.cls) else "lpql"
+        k = list_kernel_symbol(g.cls).split("_")[1]
         fam[k] = fam.get(k, 0.0) + ms
     res["eager_class_ms"] = {"total": sum(ms for ms, _ in per), "by_family": fam,
                              "note": "classes one after another on one stream, per-class events"}

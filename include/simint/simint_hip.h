@@ -229,12 +229,14 @@ const char *simint_hip_last_error(void);
 /* Kernel family used for a class: 1 = lane-per-quartet (registers),
  * 2 = wave-per-quartet (LDS-staged), 3 / 4 = split lane-per-quartet (the
  * contracted HRR inputs processed in groups of about 64 / 128, through a
- * device staging area), 0 = class not built.  The setter lets a caller (the
+ * device staging area), 5 / 6 = the same over ket tops, 7 = component-lane
+ * (one lane per component of the wider side), 0 = class not built.  The setter lets a caller (the
  * autotuner, tests) pick a family; it returns the previous one or a
  * negative value if that family is not built for the class. */
 int simint_hip_class_kernel(int la, int lb, int lc, int ld);
 int simint_hip_set_class_kernel(int la, int lb, int lc, int ld, int family);
-/* The same for the quartet-list calls: 1 = lane-per-quartet, 2 = wave-per-quartet. */
+/* The same for the quartet-list calls: 1 = lane-per-quartet, 2 = wave-per-quartet,
+ * 7 = component-lane. */
 int simint_hip_class_list_kernel(int la, int lb, int lc, int ld);
 int simint_hip_set_class_list_kernel(int la, int lb, int lc, int ld, int family);
 

@@ -3,9 +3,10 @@
 For every class, times each kernel family built for it -- lane-per-quartet
 (registers), wave-per-quartet (LDS-staged, batched), the split
 lane-per-quartet kernels with two group counts and, for bra-heavy d
-classes, their ket-top-group variants -- on the screened quartets
-of a synthetic system built with the 64-atom benchmark recipe at a smaller
-size, and writes the fastest family per class to tuning.json (read by the
+classes, their ket-top-group variants, and the component-lane kernels -- on
+the screened quartets of a synthetic system built with the 64-atom benchmark
+recipe at a smaller size (classes that system does not have: on random shell
+pairs of depth 1-3 in an 8-bohr cube), and writes the fastest family per class to tuning.json (read by the
 build to set each class's default):
 
     python simint-generator_amd/autotune.py [--natom 16] [--reps 3] [--out PATH]
@@ -60,7 +61,8 @@ def main():
         name = quartets.simint_class_name(cls)
         prev = L.simint_hip_class_kernel(*cls)
         res = {}
-        for fam, fname in ((1, "lpq"), (2, "wpq"), (3, "lpqs_a"), (4, "lpqs_b"), (5, "lpqsf_a"), (6, "lpqsf_b")):
+        for fam, fname in ((1, "lpq"), (2, "wpq"), (3, "lpqs_a"), (4, "lpqs_b"), (5, "lpqsf_a"), (6, "lpqsf_b"),
+                           (7, "cpl")):
             if L.simint_hip_set_class_kernel(*cls, fam) < 0:
                 continue
             best = None
@@ -81,13 +83,74 @@ def main():
             family[name] = min(res, key=res.get)
             timings[name] = res
             print("%-8s %s" % (name, "  ".join("%s %.3f ms" % kv for kv in sorted(res.items()))), flush=True)
+    tune_other(a, family, timings)
     doc = json.load(open(a.out)) if os.path.exists(a.out) else {}
-    doc.update({"workload": "64-atom recipe, %d atoms, Schwarz 1e-12, quartets of each class" % a.natom,
+    doc.update({"workload": "64-atom recipe, %d atoms, Schwarz 1e-12, quartets of each class; "
+                "the other classes: 96 x 512 random pairs of depth 1-3" % a.natom,
                 "family": family, "timings_ms": timings,
                 "generated": time.strftime("%Y-%m-%d %H:%M:%S")})
     with open(a.out, "w") as f:
         json.dump(doc, f, indent=1, sort_keys=True)
     print("wrote", a.out)
+
+
+def tune_other(a, family, timings):
+    """Prefix-kernel family of the classes up to f that the molecule recipe
+    has none of: 96 bra against 512 ket pairs of shells of depth 1-3 with
+    exponents log-uniform in [0.1, 50] in an 8-bohr cube."""
+    import itertools
+    import numpy as np
+    import torch
+    import quartets
+    import simint
+    L = simint.lib()
+    rng = np.random.default_rng(0)
+    shells = []
+    for l in range(4):
+        for _ in range(64):
+            k = int(rng.integers(1, 4))
+            shells.append((l, tuple(rng.uniform(0, 8, 3)), list(np.exp(rng.uniform(np.log(0.1), np.log(50), k))),
+                           list(rng.uniform(0.1, 1.0, k))))
+    basis = simint.Basis(shells)
+    stream = torch.cuda.ExternalStream(L.simint_hip_stream())
+    sets = {}
+    for la, lb in itertools.product(range(4), repeat=2):
+        for n in (96, 512):
+            pr = [(64 * la + int(i), 64 * lb + int(j)) for i, j in rng.integers(0, 64, (n, 2))]
+            pr.sort(key=lambda p: -len(shells[p[0]][2]) * len(shells[p[1]][2]))
+            hp = simint.Pairs.from_pairs(basis, pr)
+            sets[la, lb, n] = simint.DevicePairs(hp)
+            hp.free()
+    out = torch.empty(96 * 512 * 10000, dtype=torch.float64, device="cuda")
+    for cls in itertools.product(range(4), repeat=4):
+        name = quartets.simint_class_name(cls)
+        if name in family:
+            continue
+        P, Q = sets[cls[0], cls[1], 96], sets[cls[2], cls[3], 512]
+        nc = int(np.prod([simint.ncart(l) for l in cls]))
+        nket = np.full(96, 512, dtype=np.int32)
+        off = np.arange(96, dtype=np.int64) * 512 * nc
+        prev = L.simint_hip_class_kernel(*cls)
+        res = {}
+        for fname, fam in simint.FAMILIES.items():
+            if L.simint_hip_set_class_kernel(*cls, fam) < 0:
+                continue
+            for rep in range(a.reps + 1):
+                e0 = torch.cuda.Event(enable_timing=True)
+                e1 = torch.cuda.Event(enable_timing=True)
+                e0.record(stream)
+                simint.compute_prefix(P, Q, 0, nket, off, out.data_ptr())
+                e1.record(stream)
+                simint.synchronize()
+                if rep > 0:
+                    res[fname] = min(res.get(fname, 1e30), e0.elapsed_time(e1))
+        L.simint_hip_set_class_kernel(*cls, prev)
+        family[name] = min(res, key=res.get)
+        timings[name] = res
+        print("%-8s %s" % (name, "  ".join("%s %.3f ms" % kv for kv in sorted(res.items()))), flush=True)
+    for d in sets.values():
+        d.free()
+    basis.free()
 
 
 def tune_lists(a):
@@ -108,7 +171,7 @@ def tune_lists(a):
         name = "_".join("spdfghik"[x] for x in g.cls)
         prev = L.simint_hip_class_list_kernel(*g.cls)
         res = {}
-        for fam, fname in ((1, "lpq"), (2, "wpq")):
+        for fam, fname in ((1, "lpq"), (2, "wpq"), (7, "cpl")):
             if L.simint_hip_set_class_list_kernel(*g.cls, fam) < 0:
                 continue
             best = None

@@ -110,12 +110,13 @@ def build(maxam=DEFAULT_MAXAM, jobs=None, verbose=True):
         d = json.load(open(okf))
         if d.get("maxam") == maxam:
             lpq_ok = set(tuple(x) for x in d["ok"])
-    lpq, wpq, sel, lpqs = gen_mod.generate(PKG, INCLUDE, maxam, lpq_ok)
+    lpq, wpq, sel, lpqs, cpl = gen_mod.generate(PKG, INCLUDE, maxam, lpq_ok)
     hdr = _header_hash()
     srcs = sorted(glob.glob(os.path.join(GEN, "eri_*.hip")))
     # drop stale generated kernels of classes outside this build
     from emitter.hip_lpq import class_name
     want = set("eri_lpq_%s.hip" % class_name(a) for a in lpq) | set("eri_wpq_%s.hip" % class_name(a) for a in wpq)
+    want |= set("eri_cpl_%s.hip" % class_name(a) for a in cpl)
     from emitter.hip_lpqs import kernel_name
     # split kernels: keys (a,b,c,d) for the default kind, ("f", a,b,c,d) for
     # the ket-top variants of bra-heavy classes
@@ -146,7 +147,7 @@ def build(maxam=DEFAULT_MAXAM, jobs=None, verbose=True):
             ok.add(am)
     with open(okf, "w") as f:
         json.dump({"maxam": maxam, "ok": sorted(list(a) for a in ok)}, f)
-    lpq, wpq, sel, lpqs = gen_mod.generate(PKG, INCLUDE, maxam, ok)
+    lpq, wpq, sel, lpqs, cpl = gen_mod.generate(PKG, INCLUDE, maxam, ok)
     hdr = _header_hash()
     dobj, _, built = _compile_dispatch(hdr)
     objs["dispatch"] = dobj

@@ -3,6 +3,7 @@
   boys_grid.inc, boys_longfac.inc   Boys tables (emitter/boys_table.py)
   eri_lpq_<class>.hip               lane-per-quartet kernels (hip_lpq.py)
   eri_wpq_<class>.hip               wave-per-quartet kernels (hip_wpq.py)
+  eri_cpl_<class>.hip               component-lane kernels (hip_cpl.py)
   eri_lpqs<G>_<class>.hip           split lane-per-quartet kernels, G bra-top
                                     groups (hip_lpqs.py)
   dispatch.cpp                      launcher tables + kernel-family choice
@@ -15,14 +16,15 @@ import itertools
 import json
 import os
 
-from . import boys_table, config_header, hip_lpq, hip_lpqs, hip_wpq
+from . import boys_table, config_header, hip_cpl, hip_lpq, hip_lpqs, hip_wpq
 from .rrgraph import graph, ncart
 
 # Lane-per-quartet kernels are built for every class.  The default family
 # per class is lane-per-quartet when the compiler reports no scratch spills,
 # else the split lane-per-quartet kernel where one is built, else
-# wave-per-quartet; tuning.json (written by autotune.py from GPU timings)
-# overrides the default.
+# wave-per-quartet (derivative terms with a g shell: component-lane);
+# tuning.json (written by autotune.py from GPU timings of every family a
+# class has) overrides the default.
 # (the register kernels of the largest f classes are left out: their
 # straight-line code runs to >10^5 statements and could only spill)
 LPQ_MAX_TOPS = 1000
@@ -78,9 +80,9 @@ def deriv_term_classes(maxam):
     """Classes with one AM of maxam+1 that first derivatives of classes up to
     maxam need: the (a+1) terms of every centre but the first with the
     highest AM (ostei_deriv1_generator.cpp:96-124).  They run the
-    cooperative kernels, whose work area fits the local data share for
-    every one of them (the largest, (ff|fg) and its permutations, take
-    146 KB)."""
+    component-lane kernels (the cooperative kernels are built for them too;
+    a stream of 1500 first derivatives took 1220 ms with those, 137 ms with
+    these)."""
     out = set()
     for am in itertools.product(range(maxam + 1), repeat=4):
         skip = am.index(max(am))
@@ -129,7 +131,7 @@ def mixed_candidate(am):
     return max(am) <= MIXED_MAXAM
 
 
-def dispatch_text(maxam, lpq, wpq, selection, lpqs=None, list_selection=None, lpqsf=None):
+def dispatch_text(maxam, lpq, wpq, selection, lpqs=None, list_selection=None, lpqsf=None, cpl=()):
     # tables reach one AM above the maximum when derivative terms are built
     n = 1 + max(max(am) for am in wpq)
     lines = ["// Generated by simint-generator_amd/emitter/generate.py -- do not edit.",
@@ -160,6 +162,10 @@ def dispatch_text(maxam, lpq, wpq, selection, lpqs=None, list_selection=None, lp
                          % hip_lpqs.kernel_name(am, G, "f"))
     for am in wpq:
         lines.append('extern "C" hipError_t simint_launch_wpql_%s(const EriListArgs *, hipStream_t);'
+                     % hip_lpq.class_name(am))
+    for am in cpl:
+        lines.append('extern "C" hipError_t simint_launch_cpl_%s(const EriArgs *, hipStream_t);' % hip_lpq.class_name(am))
+        lines.append('extern "C" hipError_t simint_launch_cpll_%s(const EriListArgs *, hipStream_t);'
                      % hip_lpq.class_name(am))
     lines.append("")
     lines.append("namespace {")
@@ -209,6 +215,8 @@ def dispatch_text(maxam, lpq, wpq, selection, lpqs=None, list_selection=None, lp
     table("g_stage_f", None, None, typ="int",
           cell=lambda am: str(hip_lpqs.staging_doubles(am, "f") if lpqsf.get(am) else 0))
     table("g_wpql", set(wpq), "wpql", "simint_list_launch_fn")
+    table("g_cpl", set(cpl), "cpl")
+    table("g_cpll", set(cpl), "cpll", "simint_list_launch_fn")
     flat = []
     for am in itertools.product(range(n), repeat=4):
         flat.append(str(selection.get(am, 0)))
@@ -232,6 +240,7 @@ def dispatch_text(maxam, lpq, wpq, selection, lpqs=None, list_selection=None, lp
     lines.append("    if (s == 4) return g_lpqs_b[la][lb][lc][ld];")
     lines.append("    if (s == 5) return g_lpqs_c[la][lb][lc][ld];")
     lines.append("    if (s == 6) return g_lpqs_d[la][lb][lc][ld];")
+    lines.append("    if (s == 7) return g_cpl[la][lb][lc][ld];")
     lines.append("    return nullptr;")
     lines.append("}")
     lines.append("")
@@ -255,6 +264,7 @@ def dispatch_text(maxam, lpq, wpq, selection, lpqs=None, list_selection=None, lp
     lines.append("    if (!in_range(la, lb, lc, ld)) return nullptr;")
     lines.append("    const int s = g_sel_list[idx(la, lb, lc, ld)].load(std::memory_order_relaxed);")
     lines.append("    if (s == 1 && g_lpql[la][lb][lc][ld]) return g_lpql[la][lb][lc][ld];")
+    lines.append("    if (s == 7 && g_cpll[la][lb][lc][ld]) return g_cpll[la][lb][lc][ld];")
     lines.append("    return g_wpql[la][lb][lc][ld];")
     lines.append("}")
     lines.append("")
@@ -269,7 +279,8 @@ def dispatch_text(maxam, lpq, wpq, selection, lpqs=None, list_selection=None, lp
     lines.append("    if (!in_range(la, lb, lc, ld)) return -1;")
     lines.append("    if (family == 1 && !g_lpql[la][lb][lc][ld]) return -1;")
     lines.append("    if (family == 2 && !g_wpql[la][lb][lc][ld]) return -1;")
-    lines.append("    if (family < 1 || family > 2) return -1;")
+    lines.append("    if (family == 7 && !g_cpll[la][lb][lc][ld]) return -1;")
+    lines.append("    if (family != 1 && family != 2 && family != 7) return -1;")
     lines.append("    return g_sel_list[idx(la, lb, lc, ld)].exchange(family);")
     lines.append("}")
     lines.append("")
@@ -288,13 +299,14 @@ def dispatch_text(maxam, lpq, wpq, selection, lpqs=None, list_selection=None, lp
     lines.append("    if (family == 4 && !g_lpqs_b[la][lb][lc][ld]) return -1;")
     lines.append("    if (family == 5 && !g_lpqs_c[la][lb][lc][ld]) return -1;")
     lines.append("    if (family == 6 && !g_lpqs_d[la][lb][lc][ld]) return -1;")
-    lines.append("    if (family < 1 || family > 6) return -1;")
+    lines.append("    if (family == 7 && !g_cpl[la][lb][lc][ld]) return -1;")
+    lines.append("    if (family < 1 || family > 7) return -1;")
     lines.append("    return g_sel[idx(la, lb, lc, ld)].exchange(family);")
     lines.append("}")
     return "\n".join(lines) + "\n"
 
 
-FAMILIES = {"lpq": 1, "wpq": 2, "lpqs_a": 3, "lpqs_b": 4, "lpqsf_a": 5, "lpqsf_b": 6}
+FAMILIES = {"lpq": 1, "wpq": 2, "lpqs_a": 3, "lpqs_b": 4, "lpqsf_a": 5, "lpqsf_b": 6, "cpl": 7}
 
 
 def load_tuning(pkg_root, key="family"):
@@ -313,7 +325,7 @@ def load_tuning(pkg_root, key="family"):
 def generate(pkg_root, include_root, maxam, lpq_ok=None):
     """Write generated sources.  lpq_ok: set of classes whose LPQ build was
     spill-free (None = before the first compile: every candidate counts).
-    Returns (lpq_classes, wpq_classes, selection)."""
+    Returns (lpq_classes, wpq_classes, selection, split groups, cpl_classes)."""
     gen = os.path.join(pkg_root, "csrc", "gen")
     os.makedirs(gen, exist_ok=True)
     boys_table.write(gen)
@@ -326,6 +338,9 @@ def generate(pkg_root, include_root, maxam, lpq_ok=None):
                hip_lpq.emit_lpq(am, mixed=mixed_candidate(am)))
     for am in wpq:
         _write(os.path.join(gen, "eri_wpq_%s.hip" % hip_lpq.class_name(am)), hip_wpq.emit_wpq(am))
+    cpl = [am for am in wpq if hip_cpl.candidate(am)]
+    for am in cpl:
+        _write(os.path.join(gen, "eri_cpl_%s.hip" % hip_lpq.class_name(am)), hip_cpl.emit_cpl(am))
     lpqs = {}
     for am in cls:
         Gs = lpqs_variants(am)
@@ -345,6 +360,8 @@ def generate(pkg_root, include_root, maxam, lpq_ok=None):
     tuned = load_tuning(pkg_root)
 
     def built(am, fam):
+        if fam == 7:
+            return am in cpl
         if fam < 3:
             return True
         if fam < 5:
@@ -360,17 +377,18 @@ def generate(pkg_root, include_root, maxam, lpq_ok=None):
         else:
             selection[am] = 2
     for am in gterms:
-        selection[am] = 2
+        selection[am] = 7 if am in cpl else 2
     list_sel = {}
     tuned_list = load_tuning(pkg_root, "list_family")
     for am in cls:
-        if am in tuned_list and tuned_list[am] in (1, 2) and (tuned_list[am] == 2 or am in lpq):
+        if am in tuned_list and tuned_list[am] in (1, 2, 7) and (tuned_list[am] == 2 or am in (lpq if tuned_list[am] == 1
+                                                                                              else cpl)):
             list_sel[am] = tuned_list[am]
         elif am in lpq and (lpq_ok is None or am in lpq_ok):
             list_sel[am] = 1
         else:
             list_sel[am] = 2
-    _write(os.path.join(gen, "dispatch.cpp"), dispatch_text(maxam, lpq, wpq, selection, lpqs, list_sel, lpqsf))
+    _write(os.path.join(gen, "dispatch.cpp"), dispatch_text(maxam, lpq, wpq, selection, lpqs, list_sel, lpqsf, cpl))
     fname = {v: k for k, v in FAMILIES.items()}
     info = {hip_lpq.class_name(am): dict(class_info(am), kernel=fname[selection[am]], split_groups=lpqs.get(am, []),
                                          split_kernels=[hip_lpqs.kernel_name(am, G) for G in lpqs.get(am, [])],
@@ -382,4 +400,4 @@ def generate(pkg_root, include_root, maxam, lpq_ok=None):
            config_header.text(maxam, 1, maxam if gterms else maxam - 1))
     allsplit = dict(lpqs)
     allsplit.update({("f",) + am: Gs for am, Gs in lpqsf.items()})
-    return lpq, wpq, selection, allsplit
+    return lpq, wpq, selection, allsplit, cpl

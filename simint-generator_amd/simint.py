@@ -329,7 +329,7 @@ class DevicePairs:
             self.h = None
 
 
-FAMILIES = {"lpq": 1, "wpq": 2, "lpqs_a": 3, "lpqs_b": 4, "lpqsf_a": 5, "lpqsf_b": 6}
+FAMILIES = {"lpq": 1, "wpq": 2, "lpqs_a": 3, "lpqs_b": 4, "lpqsf_a": 5, "lpqsf_b": 6, "cpl": 7}
 
 
 _LIST_SPLIT = None   # class name -> lanes per quartet of its list launches
