@@ -388,6 +388,8 @@ def generate(pkg_root, include_root, maxam, lpq_ok=None):
             list_sel[am] = 1
         else:
             list_sel[am] = 2
+    for am in gterms:
+        list_sel[am] = selection[am]
     _write(os.path.join(gen, "dispatch.cpp"), dispatch_text(maxam, lpq, wpq, selection, lpqs, list_sel, lpqsf, cpl))
     fname = {v: k for k, v in FAMILIES.items()}
     info = {hip_lpq.class_name(am): dict(class_info(am), kernel=fname[selection[am]], split_groups=lpqs.get(am, []),
