@@ -9,7 +9,8 @@
 //     data share; every lane then forms its own Cartesian products
 //     S_x S_y S_z (T_x S_y S_z + S_x T_y S_z + S_x S_y T_z) and accumulates
 //     them, times c_a c_b, in registers;
-//   * potential: the lanes fill the Obara-Saika nuclear-attraction blocks
+//   * potential of shells up to d: osoei_potential_direct, a recurrence per
+//     lane; of higher ones: the lanes fill the Obara-Saika nuclear-attraction blocks
 //     Theta^(m)_{i,j} block by block (first centre up from the Boys values,
 //     then the second centre), each block's (m, component) entries spread
 //     over the lanes, and accumulate -Z c_a c_b Theta^(0)_{la,lb}.
@@ -250,6 +251,7 @@ __global__ void __launch_bounds__(64) osoei_potential(const OeiArgs a)
     for (long long pr = blockIdx.x; pr < a.npair; pr += gridDim.x) {
         const int A = a.pairs[2 * pr], B = a.pairs[2 * pr + 1];
         const int am1 = a.am[A], am2 = a.am[B], L = am1 + am2;
+        if (am1 <= 2 && am2 <= 2) continue;   // osoei_potential_direct's
         const int nc1 = oei_nc(am1), nc2 = oei_nc(am2), nout = nc1 * nc2;
         __syncthreads();   // the previous pair's last reads of boff are done
         if (lane == 0) {
@@ -370,13 +372,190 @@ __global__ void __launch_bounds__(64) osoei_potential(const OeiArgs a)
     }
 }
 
+// Nuclear attraction of shells up to d, one wavefront per shell pair with
+// the lanes over (primitive pair, charge): a lane runs its own recurrence in
+// registers (every index below is a constant once unrolled) and sums its
+// share, and the 64 shares are added through the local data share.  The
+// block kernel above spends a wavefront on one (primitive pair, charge), the
+// Boys function and the Gaussian product 64 times over, and a barrier per
+// block: 19.98 ms for the 73920 pairs and 64 charges of the 64-atom grid
+// molecule, bound by latency and repeated work; this one is bound by FP64
+// issue (0.28 ms).
+constexpr int OEI_DIRECT_MAXL = 2;
+constexpr int OEI_PRIMS = 32;    // primitive pairs prepared at a time
+constexpr int OEI_PVALS = 13;    // p, 1/2p, 2 pi/p e, PA, PB, P, c_a c_b
+
+constexpr OeiCartTable kOeiC = oei_make_table();
+
+template <int LA, int LB>
+__device__ __forceinline__ void potential_add(const double *grid, const double *v, const double *C, double Z,
+                                              double *acc)
+{
+    constexpr int L = LA + LB;
+    const double p = v[0], oo2p = v[1], pre = v[2];
+    const double PA[3] = {v[3], v[4], v[5]}, PB[3] = {v[6], v[7], v[8]};
+    const double PC[3] = {v[9] - C[0], v[10] - C[1], v[11] - C[2]};
+    double F[L + 1];
+    boys_eval<L>(grid, (PC[0] * PC[0] + PC[1] * PC[1] + PC[2] * PC[2]) * p, F);
+    // th[i][j][component of i][of j][m]; (i,0) keeps m <= L - i, (i,j>0) m <= LB - j
+    double th[LA + 1][LB + 1][oei_nc(LA)][oei_nc(LB)][L + 1];
+#pragma unroll
+    for (int m = 0; m <= L; m++) th[0][0][0][0][m] = F[m] * pre;
+#pragma unroll
+    for (int i = 0; i <= LA; i++) {
+        if (i > 0) {
+#pragma unroll
+            for (int n = 0; n < oei_nc(i); n++) {
+                const OeiCart &c = kOeiC.c[i][n];
+                const int d = c.dir;
+#pragma unroll
+                for (int m = 0; m <= L - i; m++) {
+                    const double *w1 = th[i - 1][0][c.dn1[d]][0];
+                    double t = PA[d] * w1[m] - PC[d] * w1[m + 1];
+                    if (c.e[d] > 1) {
+                        const double *w2 = th[i > 1 ? i - 2 : 0][0][c.dn2[d] < 0 ? 0 : c.dn2[d]][0];
+                        t += oo2p * (c.e[d] - 1) * (w2[m] - w2[m + 1]);
+                    }
+                    th[i][0][n][0][m] = t;
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 1; j <= LB; j++) {
+#pragma unroll
+            for (int n = 0; n < oei_nc(i); n++) {
+#pragma unroll
+                for (int o = 0; o < oei_nc(j); o++) {
+                    const OeiCart &c = kOeiC.c[j][o];
+                    const int d = c.dir;
+                    const int ei = kOeiC.c[i][n].e[d], i1 = c.dn1[d];
+#pragma unroll
+                    for (int m = 0; m <= LB - j; m++) {
+                        const double *w1 = th[i][j - 1][n][i1];
+                        double t = PB[d] * w1[m] - PC[d] * w1[m + 1];
+                        if (ei > 0) {
+                            const double *w2 = th[i > 0 ? i - 1 : 0][j - 1][ei > 0 ? kOeiC.c[i][n].dn1[d] : 0][i1];
+                            t += oo2p * ei * w2[m] - oo2p * ei * w2[m + 1];
+                        }
+                        if (c.e[d] > 1) {
+                            const double *w3 = th[i][j > 1 ? j - 2 : 0][n][c.dn2[d] < 0 ? 0 : c.dn2[d]];
+                            t += oo2p * (c.e[d] - 1) * (w3[m] - w3[m + 1]);
+                        }
+                        th[i][j][n][o][m] = t;
+                    }
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < oei_nc(LA); n++)
+#pragma unroll
+        for (int o = 0; o < oei_nc(LB); o++) acc[n * oei_nc(LB) + o] -= th[LA][LB][n][o][0] * Z * v[12];
+}
+
+// one pair: lanes over (primitive pair, charge) in batches of OEI_PRIMS
+// primitive pairs, then the lanes' sums, 16 components at a time
+template <int LA, int LB>
+__device__ __forceinline__ void potential_pair(const OeiArgs &a, int A, int B, long long off, double *prim, double *red)
+{
+    constexpr int NOUT = oei_nc(LA) * oei_nc(LB);
+    const int lane = threadIdx.x;
+    const int npa = a.nprim[A], npb = a.nprim[B], K = npa * npb;
+    const double xa[3] = {a.xyz[3 * A], a.xyz[3 * A + 1], a.xyz[3 * A + 2]};
+    const double xb[3] = {a.xyz[3 * B], a.xyz[3 * B + 1], a.xyz[3 * B + 2]};
+    const double AB[3] = {xa[0] - xb[0], xa[1] - xb[1], xa[2] - xb[2]};
+    const double AB2 = AB[0] * AB[0] + AB[1] * AB[1] + AB[2] * AB[2];
+    double acc[NOUT];
+#pragma unroll
+    for (int k = 0; k < NOUT; k++) acc[k] = 0.0;
+    for (int k0 = 0; k0 < K; k0 += OEI_PRIMS) {
+        const int nk = K - k0 < OEI_PRIMS ? K - k0 : OEI_PRIMS;
+        __syncthreads();   // the last batch's (or pair's) reads are done
+        if (lane < nk) {
+            const int ia = (k0 + lane) / npb, ib = k0 + lane - ia * npb;
+            const double a1 = a.alpha[a.poff[A] + ia], a2 = a.alpha[a.poff[B] + ib];
+            const double oop = 1.0 / (a1 + a2);
+            const double mu = a1 * a2 * oop;
+            double *v = prim + lane * OEI_PVALS;
+            v[0] = a1 + a2;
+            v[1] = 0.5 * oop;
+            v[2] = 2 * kPi * oop * exp(-mu * AB2);
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                const double P = (a1 * xa[d] + a2 * xb[d]) * oop;
+                v[3 + d] = P - xa[d];
+                v[6 + d] = P - xb[d];
+                v[9 + d] = P;
+            }
+            v[12] = a.coef[a.poff[A] + ia] * a.coef[a.poff[B] + ib];
+        }
+        __syncthreads();
+        // charges of one primitive pair side by side
+        const long long n = (long long)nk * a.ncenter;
+        for (long long t = lane; t < n; t += 64) {
+            const int k = n < (1LL << 31) ? (int)((unsigned)t / (unsigned)a.ncenter) : (int)(t / a.ncenter);
+            const double *q = a.charges + 4 * (t - (long long)k * a.ncenter);
+            const double C[3] = {q[1], q[2], q[3]};
+            potential_add<LA, LB>(a.boys, prim + k * OEI_PVALS, C, q[0], acc);
+        }
+    }
+    // lane l sums component l % 16 over the lanes 16 (l / 16) .. + 15
+#pragma unroll
+    for (int k0 = 0; k0 < NOUT; k0 += 16) {
+        __syncthreads();
+#pragma unroll
+        for (int k = k0; k < NOUT && k < k0 + 16; k++) red[(k - k0) * 65 + lane] = acc[k];
+        __syncthreads();
+        const int k = lane & 15;
+        double s = 0.0;
+        if (k0 + k < NOUT)
+            for (int l = 0; l < 16; l++) s += red[k * 65 + (lane >> 4) * 16 + l];
+        s += __shfl_xor(s, 16);
+        s += __shfl_xor(s, 32);
+        if (lane < 16 && k0 + k < NOUT) a.out[off + k0 + k] = s;
+    }
+}
+
+// pairs of shells up to d: HEAVY takes (p|d), (d|p) and (d|d) (about 250
+// registers), the other kernel the rest; a pair of the other kernel's, or
+// with a higher shell, is left alone
+template <bool HEAVY>
+__global__ void __launch_bounds__(64) osoei_potential_direct(const OeiArgs a)
+{
+    __shared__ double prim[OEI_PRIMS * OEI_PVALS];
+    __shared__ double red[16 * 65];
+    for (long long pr = blockIdx.x; pr < a.npair; pr += gridDim.x) {
+        const int A = a.pairs[2 * pr], B = a.pairs[2 * pr + 1];
+        const int la = a.am[A], lb = a.am[B];
+        const long long off = a.off[pr];
+        if (la > OEI_DIRECT_MAXL || lb > OEI_DIRECT_MAXL || (la + lb > 2) != HEAVY) continue;
+        if constexpr (HEAVY) {
+            if (la == 1) potential_pair<1, 2>(a, A, B, off, prim, red);
+            else if (lb == 1) potential_pair<2, 1>(a, A, B, off, prim, red);
+            else potential_pair<2, 2>(a, A, B, off, prim, red);
+        } else {
+            if (la == 0 && lb == 0) potential_pair<0, 0>(a, A, B, off, prim, red);
+            else if (la == 0 && lb == 1) potential_pair<0, 1>(a, A, B, off, prim, red);
+            else if (la == 1 && lb == 0) potential_pair<1, 0>(a, A, B, off, prim, red);
+            else if (la == 1) potential_pair<1, 1>(a, A, B, off, prim, red);
+            else if (la == 0) potential_pair<0, 2>(a, A, B, off, prim, red);
+            else potential_pair<2, 0>(a, A, B, off, prim, red);
+        }
+    }
+}
+
 template <int MAXL>
-hipError_t launch_osoei(int kind, const OeiArgs &a, hipStream_t s)
+hipError_t launch_osoei(int kind, int maxam, const OeiArgs &a, hipStream_t s)
 {
     const unsigned grid = (unsigned)std::min<long long>(a.npair, 1 << 20);
     if (kind == 0) hipLaunchKernelGGL((osoei_sk<0, MAXL>), dim3(grid), dim3(64), 0, s, a);
     else if (kind == 1) hipLaunchKernelGGL((osoei_sk<1, MAXL>), dim3(grid), dim3(64), 0, s, a);
-    else hipLaunchKernelGGL((osoei_potential<MAXL>), dim3(grid), dim3(64), 0, s, a);
+    else {
+        // every pair belongs to exactly one of these
+        hipLaunchKernelGGL((osoei_potential_direct<false>), dim3(grid), dim3(64), 0, s, a);
+        if (maxam > 1) hipLaunchKernelGGL((osoei_potential_direct<true>), dim3(grid), dim3(64), 0, s, a);
+        if (maxam > OEI_DIRECT_MAXL) hipLaunchKernelGGL((osoei_potential<MAXL>), dim3(grid), dim3(64), 0, s, a);
+    }
     return hipGetLastError();
 }
 
@@ -444,7 +623,7 @@ OeiArgs shell_args(char *base, const ShellImage &im)
 
 hipError_t launch_any(int kind, int maxam, const OeiArgs &a, hipStream_t s)
 {
-    return maxam <= 3 ? launch_osoei<3>(kind, a, s) : launch_osoei<OEI_MAXL>(kind, a, s);
+    return maxam <= 3 ? launch_osoei<3>(kind, maxam, a, s) : launch_osoei<OEI_MAXL>(kind, maxam, a, s);
 }
 
 // one pair through the calling thread's staging buffers (the drop-in calls)
