@@ -1205,12 +1205,15 @@ thread_local int t_list_split = 0;   // 0: by list length
 
 // Lanes per quartet for a lane-per-quartet list launch of n quartets: enough
 // that the launch has about 65536 lanes (a short list of one class otherwise
-// occupies a few dozen wavefronts), at most 16.
+// occupies a few dozen wavefronts), up to 16; up to a whole wavefront while
+// it has fewer than 16384 (a list of six quartets of up to 1296 primitive
+// quartets otherwise leaves 81 of them to one lane).
 int list_split(long long n)
 {
     if (t_list_split > 0) return t_list_split;
     int s = 1;
     while (s < 16 && n * s < 65536) s *= 2;
+    while (s < 64 && n * s < 16384) s *= 2;
     return s;
 }
 

@@ -290,9 +290,12 @@ def base_G(am):
 def candidate(am):
     """Classes this family is built for: a wide side of at least f in all,
     and a narrow side of at least p (the (gf|ss) derivative terms have no
-    lane-per-quartet kernel; lower (ab|ss) classes run that)."""
+    lane-per-quartet kernel; lower (ab|ss) classes run that); classes with
+    an HRR and a wide side of d for their small launches."""
     g = graph(*am)
-    if max(g.e_hi, g.f_hi) < (3 if min(g.e_hi, g.f_hi) > 0 else 7):
+    wide, narrow = max(g.e_hi, g.f_hi), min(g.e_hi, g.f_hi)
+    hrr = g.bra_hrr_needed() or g.ket_hrr_needed()
+    if wide < (7 if narrow == 0 else 2 if hrr else 3):
         return False
     try:
         plan(am, base_G(am))

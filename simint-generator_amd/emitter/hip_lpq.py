@@ -380,15 +380,144 @@ def emit_lpq(am, mixed=False):
     if mixed:
         w("")
         _emit_lpq_prefix(am, w, "float")
+    for fp in (("double", "float") if mixed else ("double",)):
+        if share_kind(am) in ("sum", "turn"):
+            _emit_lpq_prefix(am, w, fp, shared=share_kind(am))
+        _emit_lpq_launcher(am, w, fp)
     return w.text()
 
 
-def _emit_lpq_prefix(am, w, fp, hrr_fp="double"):
+# Small launches: several wavefronts share an item's primitive quartets while
+# the launch has fewer than SHARE_ITEMS wavefronts (the chip holds 4096), eight
+# at most.  A 12-atom molecule's (ss|ss) launches are a few dozen items of up
+# to 1296 primitive quartets: 82 us each with one wavefront an item, 24 us so.
+# Classes without HRR add the wavefronts' sums at the end.  An HRR amplifies
+# the rounding of another order of the sum, so the others keep the order:
+#  * (ab|ss) and (ss|cd): the wavefronts take the primitive quartets in turn,
+#    leave the contracted terms in the local data share, and every contracted
+#    value is added up by one of them in the order one wavefront alone adds it;
+#  * the rest run the component-lane kernel up to SMALL_ITEMS items, which
+#    spreads a quartet over lanes instead and gives the same values: 81
+#    primitive quartets of (dp|ps) take 196 us with one wavefront an item and
+#    78 us so for 1 item, 202 and 128 us for 128, 201 and 224 for 256.
+SHARE_ITEMS = 2048
+SMALL_ITEMS = 128
+SHARE_SUM = 8       # contracted values added per round at the end (classes without HRR)
+
+
+def share_kind(am):
+    """"sum", "turn" or "lanes" (see above); None: one wavefront an item
+    whatever the launch."""
+    from . import hip_cpl
+    g = graph(*am)
+    if not g.bra_hrr_needed() and not g.ket_hrr_needed():
+        return "sum" if len(g.top_keys) <= 128 else None
+    if min(g.e_hi, g.f_hi) == 0:
+        return "turn" if len(g.top_keys) <= 64 else None
+    return "lanes" if hip_cpl.candidate(am) else None
+
+
+def share_waves(am):
+    """Most wavefronts that share an item: "turn" keeps two buffers of their
+    terms, at most 128 KB of the local data share; "sum" leaves 256
+    registers a lane with eight, 512 with four."""
+    ntop = len(graph(*am).top_keys)
+    if share_kind(am) == "sum":
+        return 8 if ntop <= 36 else 4
+    return 8 if ntop <= 16 else 4 if ntop <= 32 else 2
+
+
+def _emit_lpq_launcher(am, w, fp):
+    kname = ("lpqm_%s" if fp == "float" else "lpq_%s") % class_name(am)
+    kind, most = share_kind(am), share_waves(am)
+    if kind == "lanes" and fp == "double":
+        w('extern "C" hipError_t simint_launch_cpl_%s(const EriArgs *a, hipStream_t s);' % class_name(am))
+    w('extern "C" hipError_t simint_launch_%s(const EriArgs *a, hipStream_t s)' % kname)
+    w("{")
+    w("    if (a->nitems <= 0) return hipSuccess;")
+    if kind == "lanes":
+        w("    if (a->nitems <= %d) return simint_launch_cpl_%s(a, s);" % (SMALL_ITEMS, class_name(am)))
+    elif kind:
+        w("    int waves = 1;")
+        w("    while (waves < %d && a->nitems * waves < %d) waves *= 2;" % (most, SHARE_ITEMS))
+        w("    if (waves > 1) {")
+        w("        hipLaunchKernelGGL(eri_%s, dim3((unsigned)a->nitems), dim3(64, waves), waves * %du, s, *a);"
+          % (kname.replace("_", "k_", 1), 2 * 512 * len(graph(*am).top_keys) if kind == "turn" else 0))
+        w("        return hipGetLastError();")
+        w("    }")
+    w("    hipLaunchKernelGGL(eri_%s, dim3((unsigned)a->nitems), dim3(64), 0, s, *a);" % kname)
+    w("    return hipGetLastError();")
+    w("}")
+    w("")
+
+
+def _emit_share_sum(ntop, most, w):
+    """Add the wavefronts' sums to the first one's, which goes on alone."""
+    w("    __shared__ double part[%d];" % ((most - 1) * SHARE_SUM * 64))
+    for v0 in range(0, ntop, SHARE_SUM):
+        vals = range(v0, min(ntop, v0 + SHARE_SUM))
+        if v0:
+            w("    __syncthreads();")
+        w("    if (wave != 0) {")
+        w("        double *const x = part + (wave - 1) * %d + lane;" % (SHARE_SUM * 64))
+        for t in vals:
+            w("        x[%d] = acc%d;" % (64 * (t - v0), t))
+        w("    }")
+        w("    __syncthreads();")
+        w("    if (wave == 0) {")
+        w("        for (int v = 0; v < waves - 1; ++v) {")
+        w("            const double *const x = part + v * %d + lane;" % (SHARE_SUM * 64))
+        for t in vals:
+            w("            acc%d += x[%d];" % (t, 64 * (t - v0)))
+        w("        }")
+        w("    }")
+    w("    if (wave != 0) return;")
+
+
+def _emit_share_turn(ntop, most, w):
+    """The round's terms of every wavefront to the local data share (two
+    buffers by turns, one barrier a round), then the owned values' sums."""
+    w("        double *const x = terms + turn * (waves * %d) + lane;" % (ntop * 64))
+    w("        turn ^= 1;")
+    for t in range(ntop):
+        w("        x[(wave * %d + %d) * 64] = acc%d;" % (ntop, t, t))
+    w("        __syncthreads();")
+    w("#pragma unroll")
+    w("        for (int k = 0; k < OWN; ++k) {")
+    w("            const int t = wave + waves * k;")
+    w("            if (t < %d) {" % ntop)
+    w("                double y[%d];   // all loads before the sum" % most)
+    w("#pragma unroll")
+    w("                for (int v = 0; v < %d; ++v) y[v] = v < waves ? x[(v * %d + t) * 64] : 0.0;" % (most, ntop))
+    w("#pragma unroll")
+    w("                for (int v = 0; v < %d; ++v) own[k] += y[v];" % most)
+    w("            }")
+    w("        }")
+
+
+def _emit_share_end(ntop, w):
+    """Every sum to the first wavefront, which goes on alone."""
+    w("    __syncthreads();")
+    w("#pragma unroll")
+    w("    for (int k = 0; k < OWN; ++k) {")
+    w("        const int t = wave + waves * k;")
+    w("        if (t < %d) terms[t * 64 + lane] = own[k];" % ntop)
+    w("    }")
+    w("    __syncthreads();")
+    w("    if (wave != 0) return;")
+    for t in range(ntop):
+        w("    const double acc%d = terms[%d + lane];" % (t, 64 * t))
+
+
+def _emit_lpq_prefix(am, w, fp, hrr_fp="double", shared=None):
+    """shared: blockDim.y wavefronts share the item's primitive quartets
+    ("sum", "turn": share_kind)."""
     g = graph(*am)
     name = class_name(am)
     ntop = len(g.top_keys)
-    kname = ("eri_lpqm_%s" if fp == "float" else "eri_lpq_%s") % name
-    w("__global__ void __launch_bounds__(64) %s(const EriArgs A)" % kname)
+    kname = ("eri_lpqm%s_%s" if fp == "float" else "eri_lpq%s_%s") % ("k" if shared else "", name)
+    most = share_waves(am)
+    w("__global__ void __launch_bounds__(%d) %s(const EriArgs A)" % (64 * most if shared else 64, kname))
     w("{")
     w("    const WorkItem wi = A.items[blockIdx.x];")
     w("    const int lane = threadIdx.x;")
@@ -399,11 +528,38 @@ def _emit_lpq_prefix(am, w, fp, hrr_fp="double"):
     w("    const long long tl = (long long)wi.tile * SIMINT_TILE + lane;")
     w("    const long long kb = A.ket.toff[wi.tile] + lane;")
     w("    const bool screen = A.tol2 > 0.0;")
-    for t in range(ntop):
-        w("    double acc%d = 0.0;" % t)
+    if shared:
+        w("    const int waves = (int)blockDim.y;")
+        w("    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.y);")
+    if shared == "sum":
+        # strides over the bra primitives and, where those are fewer, the ket's
+        w("    int istep = waves;")
+        w("    while (istep > 1 && istep > ib1 - ib0) istep >>= 1;")
+        w("    const int jstep = waves / istep;")
+        w("    const int i0 = ib0 + wave / jstep, j0 = wave % jstep;")
+    if shared == "turn":
+        w("    extern __shared__ double terms[];")
+        w("    constexpr int OWN = %d;   // values a wavefront adds up, with two of them or more" % ((ntop + 1) // 2))
+        w("    double own[OWN];")
+        w("#pragma unroll")
+        w("    for (int k = 0; k < OWN; ++k) own[k] = 0.0;")
+        w("    const int K = (ib1 - ib0) * nq;")
+        w("    int turn = 0;")
+    else:
+        for t in range(ntop):
+            w("    double acc%d = 0.0;" % t)
     bra_pa = "pa" if g.bra_j else "pb"
     ket_pa = "pa" if g.ket_l else "pb"
-    w("    for (int i = ib0; i < ib1; ++i) {")
+    if shared == "turn":
+        w("    for (int p0 = 0; p0 < K; p0 += waves) {")
+        for t in range(ntop):
+            w("        double acc%d = 0.0;" % t)
+        w("        const int p = p0 + wave;")
+        w("        const int ii = p / nq;")
+        w("        for (int once = p < K; once; once = 0) {")
+        w("        const int i = ib0 + ii, j = p - ii * nq;")
+    else:
+        w("    for (int i = i0; i < ib1; i += istep) {" if shared else "    for (int i = ib0; i < ib1; ++i) {")
     w("        const double P_alpha = A.bra.alpha[i];")
     w("        const double P_inv = A.bra.inv_alpha[i];")
     w("        const double P_prefac = A.bra.prefac[i];")
@@ -412,7 +568,8 @@ def _emit_lpq_prefix(am, w, fp, hrr_fp="double"):
       % ("PA" if g.bra_j else "PB", bra_pa, bra_pa, bra_pa))
     w("        const double P_screen = screen ? A.bra.screen[i] : 0.0;")
     w("        if (screen && P_screen * A.ket_screen_max < A.tol2) continue;")
-    w("        for (int j = 0; j < nq; ++j) {")
+    w({"turn": "        {", "sum": "        for (int j = j0; j < nq; j += jstep) {"}.get(
+        shared, "        for (int j = 0; j < nq; ++j) {"))
     w("            const long long kj = kb + (long long)SIMINT_TILE * j;")
     w("            if (screen && A.ket.screen[kj] * P_screen < A.tol2) continue;")
     w("            const double Q_alpha = A.ket.alpha[kj];")
@@ -424,6 +581,12 @@ def _emit_lpq_prefix(am, w, fp, hrr_fp="double"):
     emit_body(am, w, indent="            ", fp=fp)
     w("        }")
     w("    }")
+    if shared == "sum":
+        _emit_share_sum(ntop, most, w)
+    if shared == "turn":
+        _emit_share_turn(ntop, most, w)
+        w("    }")
+        _emit_share_end(ntop, w)
     # direct stores (through LDS slices measured 3% slower on these
     # compute-bound kernels)
     w("    if (lane < wi.lane_lo || lane >= wi.lane_hi) return;")
@@ -439,18 +602,11 @@ def _emit_lpq_prefix(am, w, fp, hrr_fp="double"):
     emit_hrr(am, w, fp=hrr_fp)
     w("}")
     w("")
-    w('extern "C" hipError_t simint_launch_%s(const EriArgs *a, hipStream_t s)' % kname[4:])
-    w("{")
-    w("    if (a->nitems <= 0) return hipSuccess;")
-    w("    hipLaunchKernelGGL(%s, dim3((unsigned)a->nitems), dim3(64), 0, s, *a);" % kname)
-    w("    return hipGetLastError();")
-    w("}")
-    w("")
 
 
 def emit_lpq_list(am, w):
     """Quartet-list variant: S = A.split lanes per quartet (a power of two
-    up to 16); lanes 64k + l take quartet (64k + l) / S, with its own bra and
+    up to 64); lanes 64k + l take quartet (64k + l) / S, with its own bra and
     ket pair (both read from the linear view, per-lane gathers).  Lane
     sub = l % S sums primitive quartets sub, sub + S, ... (bra-major order,
     as the reference's loops); the S partial sums are added across the
@@ -519,7 +675,7 @@ def emit_lpq_list(am, w):
     w('extern "C" hipError_t simint_launch_lpql_%s(const EriListArgs *a, hipStream_t s)' % name)
     w("{")
     w("    if (a->nquartet <= 0) return hipSuccess;")
-    w("    if (a->split < 1 || a->split > 16 || (a->split & (a->split - 1))) return hipErrorInvalidValue;")
+    w("    if (a->split < 1 || a->split > 64 || (a->split & (a->split - 1))) return hipErrorInvalidValue;")
     w("    hipLaunchKernelGGL(eri_lpql_%s, dim3((unsigned)((a->nquartet * a->split + 63) / 64)), dim3(64), 0, s, *a);"
       % name)
     w("    return hipGetLastError();")
