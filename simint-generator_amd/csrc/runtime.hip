@@ -211,6 +211,45 @@ struct PinBuf {
     }
 };
 
+// Pinned memory the range launches' descriptions are written to and the
+// device reads them from: two halves used in turn, each filled from its
+// start and taken again once the event recorded when it was left has passed.
+// So a launch waits only for the one that used its bytes, a half ago.
+struct PinRing {
+    struct Half {
+        PinBuf b;
+        hipEvent_t left = nullptr;
+        bool wait = false;
+    } half[2];
+    int cur = 0;
+    size_t used = 0;
+    // n bytes (256-byte aligned) on behalf of work about to be queued on s
+    hipError_t take(size_t n, hipStream_t s, char **p)
+    {
+        n = (n + 255) & ~(size_t)255;
+        hipError_t e;
+        if (used + n > half[cur].b.cap) {
+            if (used) {
+                Half &h = half[cur];
+                if (!h.left && (e = hipEventCreateWithFlags(&h.left, hipEventDisableTiming)) != hipSuccess) return e;
+                if ((e = hipEventRecord(h.left, s)) != hipSuccess) return e;
+                h.wait = true;
+                cur ^= 1;
+                used = 0;
+            }
+            Half &h = half[cur];
+            if (h.wait) {
+                if ((e = hipEventSynchronize(h.left)) != hipSuccess) return e;
+                h.wait = false;
+            }
+            if ((e = h.b.reserve(n)) != hipSuccess) return e;
+        }
+        *p = static_cast<char *>(half[cur].b.p) + used;
+        used += n;
+        return hipSuccess;
+    }
+};
+
 // Per-thread stream and buffers.  They are never released: freeing HIP
 // resources from thread-exit or static destructors can race the runtime's
 // own teardown, and the process exit returns the memory anyway.
@@ -220,10 +259,59 @@ struct ThreadCtx {
     DevBuf in, out, items;
     DevBuf split;      // staging of the split lane-per-quartet kernels
     PinBuf stage;
+    // Range launches queue without waiting for the ones before: on one
+    // stream their device buffers (items, split) are reused in order.
+    PinRing ring;
+    hipEvent_t range_ev = nullptr;
+    bool range_live = false;     // range work queued on s since s was taken up
+    bool range_marked = false;   // range_ev stands behind such work of an earlier stream
+    bool range_lost = false;     // such work was left on a stream that was being captured
     ThreadCtx()
     {
         hipStreamCreateWithFlags(&own, hipStreamNonBlocking);
         s = own;
+    }
+    // before s is left, or its work is captured: the range work queued on it
+    // ends at range_ev
+    hipError_t range_leave()
+    {
+        if (!range_live) return hipSuccess;
+        hipError_t e;
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if ((e = hipStreamIsCapturing(s, &cap)) != hipSuccess) return e;
+        if (cap != hipStreamCaptureStatusNone) {   // no event can be recorded but into the graph
+            range_live = false;
+            range_lost = true;
+            return hipSuccess;
+        }
+        if (!range_ev && (e = hipEventCreateWithFlags(&range_ev, hipEventDisableTiming)) != hipSuccess) return e;
+        if ((e = hipEventRecord(range_ev, s)) != hipSuccess) return e;
+        range_live = false;
+        range_marked = true;
+        return hipSuccess;
+    }
+    // before items or split are used on s
+    hipError_t range_enter()
+    {
+        if (range_lost) {
+            const hipError_t e = hipDeviceSynchronize();
+            if (e != hipSuccess) return e;
+            range_lost = false;
+        }
+        if (range_marked) {
+            const hipError_t e = hipStreamWaitEvent(s, range_ev, 0);
+            if (e != hipSuccess) return e;
+            range_marked = false;
+        }
+        range_live = true;
+        return hipSuccess;
+    }
+    // device memory that work queued on s may still use, grown when it must be
+    hipError_t grow(DevBuf &b, size_t n)
+    {
+        if (n <= b.cap) return hipSuccess;
+        const hipError_t e = hipStreamSynchronize(s);
+        return e != hipSuccess ? e : b.reserve(n);
     }
 };
 
@@ -766,7 +854,8 @@ int simint_compute_ostei_deriv(int deriv, const simint_multi_shellpair *P, const
     ThreadCtx &c = ctx();
     hipError_t e;
     // an earlier asynchronous call of this thread (_range, _prefix, _diag)
-    // may still read c.stage, c.in or c.split: wait for it before reuse
+    // may still read c.stage or c.split: wait for it before reuse
+    if ((e = c.range_enter()) != hipSuccess) { set_err("hipStreamWaitEvent", e); return SIMINT_ERROR_HIP; }
     if ((e = hipStreamSynchronize(c.s)) != hipSuccess) { set_err("hipStreamSynchronize", e); return SIMINT_ERROR_HIP; }
     const size_t final_n = (size_t)nP * nQ * nc * (deriv ? 12 : 1);
     const bool gamess = gamess_needed(am);
@@ -919,28 +1008,48 @@ size_t simint_hip_pairs_bytes(const simint_hip_pairs *p) { return p ? p->bytes :
 
 namespace {
 
-// items for bra b = b0 + i: its ket range [lo, hi) (lo = ket_lo[i] or 0,
-// hi = nket[i]) in tiles of 64; ket k is written at out_off[i] + (k - lo) * stride
-__global__ void expand_prefix_items(int b0, int nbra, const int *ket_lo, const int *nket,
-                                    const long long *tile_start, const long long *out_off, long long stride,
-                                    WorkItem *items)
+constexpr int kMaxTerms = 8;
+constexpr int kExpandLanes = 8;   // threads per bra
+
+// What a range launch covers, in pinned host memory: per bra its ket range,
+// its first item and, per term, its output offset.
+struct ExpandArgs {
+    int b0, nbra;
+    const int *lo, *hi;                    // lo: null for 0
+    const long long *tile_start;
+    const long long *out_off[kMaxTerms];
+    long long stride[kMaxTerms];
+    long long nitems;
+    WorkItem *items;                       // nitems per term
+    long long *tstart;                     // device copy of tile_start, or null
+};
+
+// items for bra b = b0 + i: its ket range [lo, hi) in tiles of 64; ket k is
+// written at out_off[i] + (k - lo) * stride.  Reads the ranges over PCIe
+// itself: a copy queued before it cost a short launch more than all it does.
+__global__ void __launch_bounds__(256) expand_range_items(const ExpandArgs x)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nbra) return;
-    const int lo = ket_lo ? ket_lo[i] : 0;
-    const int hi = nket[i];
-    const long long s = tile_start[i];
+    const int g = blockIdx.x * 256 + threadIdx.x;
+    const int i = g / kExpandLanes;
+    if (i >= x.nbra) return;
+    const int term = blockIdx.y;
+    const int lo = x.lo ? x.lo[i] : 0;
+    const int hi = x.hi[i];
+    const long long s = x.tile_start[i];
+    if (x.tstart && term == 0 && g % kExpandLanes == 0) x.tstart[i] = s;
     const int t0 = lo / SIMINT_TILE;
     const int nt = hi > lo ? (hi + SIMINT_TILE - 1) / SIMINT_TILE - t0 : 0;
-    for (int t = 0; t < nt; t++) {
+    const long long obase = x.out_off[term][i] - (long long)lo * x.stride[term];
+    WorkItem *items = x.items + (long long)term * x.nitems + s;
+    for (int t = g % kExpandLanes; t < nt; t += kExpandLanes) {
         WorkItem w;
-        w.bra = b0 + i;
+        w.bra = x.b0 + i;
         w.tile = t0 + t;
         w.lane_lo = max(lo - (t0 + t) * SIMINT_TILE, 0);
         w.lane_hi = min(SIMINT_TILE, hi - (t0 + t) * SIMINT_TILE);
         w.pad = 0;
-        w.obase = out_off[i] - (long long)lo * stride;
-        items[s + t] = w;
+        w.obase = obase;
+        items[t] = w;
     }
 }
 
@@ -957,8 +1066,12 @@ struct RangeTerm {
     int weight;   // -1: none
 };
 
-// items_out / nitems_out (optional): the work items of the first term, left
-// in the thread's item buffer for kernels queued after the class launch
+// items_out / nitems_out / tstart_out (optional): the work items of the first
+// term and every bra's first one, left in the thread's item buffer for
+// kernels queued after the class launch.  Returns without waiting for the
+// device: waiting for the launch before, copying the ranges and only then
+// queueing took every small launch about 40 us, more than most of its
+// kernels (a pass over 12 atoms is 253 of them).
 long long range_launch(const simint_hip_pairs *P, const simint_hip_pairs *Q, int b0, int nbra, const int *ket_lo,
                        const int *ket_hi, const long long *const *out_offs, const RangeTerm *terms, int nterm,
                        double screen_tol, double *const *d_outs, const WorkItem **items_out = nullptr,
@@ -966,61 +1079,77 @@ long long range_launch(const simint_hip_pairs *P, const simint_hip_pairs *Q, int
 {
     if (nitems_out) *nitems_out = 0;
     if (nbra == 0) return 0;
-    std::vector<long long> tstart(nbra + 1, 0);
-    long long nq = 0;
+    long long nitems = 0, nq = 0;
     for (int i = 0; i < nbra; i++) {
         const int lo = ket_lo ? ket_lo[i] : 0, hi = ket_hi[i];
         if (lo < 0 || hi > Q->n) return SIMINT_ERROR_ARGUMENT;
-        const long long nt = hi > lo ? (hi + SIMINT_TILE - 1) / SIMINT_TILE - lo / SIMINT_TILE : 0;
-        tstart[i + 1] = tstart[i] + nt;
-        nq += hi > lo ? hi - lo : 0;
+        if (hi <= lo) continue;
+        nitems += (hi + SIMINT_TILE - 1) / SIMINT_TILE - lo / SIMINT_TILE;
+        nq += hi - lo;
     }
-    const long long nitems = tstart[nbra];
     if (nitems == 0) return 0;
     ThreadCtx &c = ctx();
-    Image im;
-    const size_t o_lo = im.add(sizeof(int) * nbra);
-    const size_t o_nk = im.add(sizeof(int) * nbra);
-    const size_t o_ts = im.add(sizeof(long long) * nbra);
-    std::vector<size_t> o_oo(nterm);
-    for (int t = 0; t < nterm; t++) o_oo[t] = im.add(sizeof(long long) * nbra);
-    if (ket_lo) memcpy(im.at<int>(o_lo), ket_lo, sizeof(int) * nbra);
-    memcpy(im.at<int>(o_nk), ket_hi, sizeof(int) * nbra);
-    memcpy(im.at<long long>(o_ts), tstart.data(), sizeof(long long) * nbra);
-    for (int t = 0; t < nterm; t++) memcpy(im.at<long long>(o_oo[t]), out_offs[t], sizeof(long long) * nbra);
     hipError_t e;
-    // the previous call's kernels may still read c.in / c.items: wait for them
-    if ((e = hipStreamSynchronize(c.s)) != hipSuccess) { set_err("hipStreamSynchronize", e); return SIMINT_ERROR_HIP; }
-    if ((e = c.stage.reserve(im.buf.size())) != hipSuccess) { set_err("hipHostMalloc", e); return SIMINT_ERROR_HIP; }
-    if ((e = c.in.reserve(im.buf.size())) != hipSuccess) { set_err("hipMalloc", e); return SIMINT_ERROR_HIP; }
-    if ((e = c.items.reserve(sizeof(WorkItem) * (size_t)nitems * nterm)) != hipSuccess) {
-        set_err("hipMalloc", e);
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if ((e = hipStreamIsCapturing(c.s, &cap)) != hipSuccess) { set_err("hipStreamIsCapturing", e); return SIMINT_ERROR_HIP; }
+    if (cap != hipStreamCaptureStatusNone) {
+        // the ranges are read when the kernels run: they cannot be recorded
+        set_err("range launch", hipErrorStreamCaptureUnsupported);
         return SIMINT_ERROR_HIP;
     }
+    if ((e = c.range_enter()) != hipSuccess) { set_err("hipStreamWaitEvent", e); return SIMINT_ERROR_HIP; }
     size_t nst = 0;
     for (int t = 0; t < nterm; t++)
         nst = std::max(nst, (size_t)simint_dispatch_staging(terms[t].am[0], terms[t].am[1], terms[t].am[2],
                                                             terms[t].am[3]));
-    if (nst && (e = c.split.reserve(sizeof(double) * nst * SIMINT_TILE * (size_t)nitems)) != hipSuccess) {
+    const size_t items_bytes = sizeof(WorkItem) * (size_t)nitems * nterm;
+    if ((e = c.grow(c.items, items_bytes + sizeof(long long) * (size_t)nbra)) != hipSuccess ||
+        (e = c.grow(c.split, sizeof(double) * nst * SIMINT_TILE * (size_t)nitems)) != hipSuccess) {
         set_err("hipMalloc", e);
         return SIMINT_ERROR_HIP;
     }
-    memcpy(c.stage.p, im.buf.data(), im.buf.size());
-    if ((e = hipMemcpyAsync(c.in.p, c.stage.p, im.buf.size(), hipMemcpyHostToDevice, c.s)) != hipSuccess) {
-        set_err("hipMemcpyAsync", e);
+    // 8-byte fields first
+    const size_t n = (size_t)nbra;
+    char *host = nullptr;
+    if ((e = c.ring.take(n * (sizeof(long long) * (1 + nterm) + sizeof(int) * (ket_lo ? 2 : 1)), c.s, &host)) !=
+        hipSuccess) {
+        set_err("hipHostMalloc", e);
         return SIMINT_ERROR_HIP;
     }
-    char *base = static_cast<char *>(c.in.p);
+    long long *ts = reinterpret_cast<long long *>(host);
+    int *hi = reinterpret_cast<int *>(ts + n * (1 + nterm));
+    ExpandArgs x;
+    x.b0 = b0;
+    x.nbra = nbra;
+    x.hi = hi;
+    x.lo = nullptr;
+    x.tile_start = ts;
+    x.nitems = nitems;
+    x.items = static_cast<WorkItem *>(c.items.p);
+    x.tstart = tstart_out ? reinterpret_cast<long long *>(static_cast<char *>(c.items.p) + items_bytes) : nullptr;
+    memcpy(hi, ket_hi, sizeof(int) * n);
+    if (ket_lo) {
+        memcpy(hi + n, ket_lo, sizeof(int) * n);
+        x.lo = hi + n;
+    }
     for (int t = 0; t < nterm; t++) {
         const RangeTerm &T = terms[t];
-        WorkItem *items = static_cast<WorkItem *>(c.items.p) + (size_t)nitems * t;
-        const long long stride = (long long)ncart(T.am[0]) * ncart(T.am[1]) * ncart(T.am[2]) * ncart(T.am[3]);
-        hipLaunchKernelGGL(expand_prefix_items, dim3((nbra + 255) / 256), dim3(256), 0, c.s, b0, nbra,
-                           ket_lo ? reinterpret_cast<const int *>(base + o_lo) : (const int *)nullptr,
-                           reinterpret_cast<const int *>(base + o_nk),
-                           reinterpret_cast<const long long *>(base + o_ts),
-                           reinterpret_cast<const long long *>(base + o_oo[t]), stride, items);
-        if ((e = hipGetLastError()) != hipSuccess) { set_err("expand launch", e); return SIMINT_ERROR_HIP; }
+        long long *oo = ts + n * (1 + t);
+        memcpy(oo, out_offs[t], sizeof(long long) * n);
+        x.out_off[t] = oo;
+        x.stride[t] = (long long)ncart(T.am[0]) * ncart(T.am[1]) * ncart(T.am[2]) * ncart(T.am[3]);
+    }
+    long long at = 0;
+    for (int i = 0; i < nbra; i++) {
+        const int l = ket_lo ? ket_lo[i] : 0, h = ket_hi[i];
+        ts[i] = at;
+        if (h > l) at += (h + SIMINT_TILE - 1) / SIMINT_TILE - l / SIMINT_TILE;
+    }
+    const unsigned nblk = (unsigned)((n * kExpandLanes + 255) / 256);
+    hipLaunchKernelGGL(expand_range_items, dim3(nblk, nterm), dim3(256), 0, c.s, x);
+    if ((e = hipGetLastError()) != hipSuccess) { set_err("expand launch", e); return SIMINT_ERROR_HIP; }
+    for (int t = 0; t < nterm; t++) {
+        const RangeTerm &T = terms[t];
         EriArgs a;
         a.scratch = static_cast<double *>(c.split.p);
         a.bra = P->lin;
@@ -1029,18 +1158,18 @@ long long range_launch(const simint_hip_pairs *P, const simint_hip_pairs *Q, int
         if (T.weight == 1) a.bra.prefac = P->wb;
         if (T.weight == 2) a.ket.prefac = Q->twa;
         if (T.weight == 3) a.ket.prefac = Q->twb;
-        a.items = items;
+        a.items = x.items + nitems * t;
         a.nitems = nitems;
         a.out = d_outs[t];
         a.boys_grid = g_dev.boys;
         a.tol2 = (screen_tol > 0.0 && P->has_screen && Q->has_screen) ? screen_tol * screen_tol : 0.0;
         a.ket_screen_max = Q->screen_max;
-        a.stride = stride;
+        a.stride = x.stride[t];
         if ((e = T.fn(&a, c.s)) != hipSuccess) { set_err("class kernel launch", e); return SIMINT_ERROR_HIP; }
     }
-    if (items_out) *items_out = static_cast<const WorkItem *>(c.items.p);
+    if (items_out) *items_out = x.items;
     if (nitems_out) *nitems_out = nitems;
-    if (tstart_out) *tstart_out = reinterpret_cast<const long long *>(base + o_ts);
+    if (tstart_out) *tstart_out = x.tstart;
     return nq;
 }
 
@@ -1113,6 +1242,7 @@ long long simint_hip_compute_eri_diag(const simint_hip_pairs *P, double *d_out)
         items[b].obase = 0;
     }
     hipError_t e;
+    if ((e = c.range_enter()) != hipSuccess) { set_err("hipStreamWaitEvent", e); return SIMINT_ERROR_HIP; }
     if ((e = hipStreamSynchronize(c.s)) != hipSuccess) { set_err("hipStreamSynchronize", e); return SIMINT_ERROR_HIP; }
     const size_t bytes = sizeof(WorkItem) * items.size();
     if ((e = c.stage.reserve(bytes)) != hipSuccess) { set_err("hipHostMalloc", e); return SIMINT_ERROR_HIP; }
@@ -1412,7 +1542,9 @@ struct simint_hip_graph {
 int simint_hip_capture_begin(void)
 {
     if (!ensure_device()) return SIMINT_ERROR_NO_DEVICE;
-    hipError_t e = hipStreamBeginCapture(ctx().s, hipStreamCaptureModeThreadLocal);
+    hipError_t e = ctx().range_leave();
+    if (e != hipSuccess) { set_err("hipEventRecord", e); return SIMINT_ERROR_HIP; }
+    e = hipStreamBeginCapture(ctx().s, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) { set_err("hipStreamBeginCapture", e); return SIMINT_ERROR_HIP; }
     return 0;
 }
@@ -1477,7 +1609,12 @@ int simint_hip_set_stream(void *stream)
 {
     if (!ensure_device()) return SIMINT_ERROR_NO_DEVICE;
     ThreadCtx &c = ctx();
-    c.s = stream ? static_cast<hipStream_t>(stream) : c.own;
+    const hipStream_t to = stream ? static_cast<hipStream_t>(stream) : c.own;
+    if (to != c.s) {
+        const hipError_t e = c.range_leave();
+        if (e != hipSuccess) { set_err("hipEventRecord", e); return SIMINT_ERROR_HIP; }
+    }
+    c.s = to;
     return 0;
 }
 

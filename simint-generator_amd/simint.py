@@ -105,7 +105,8 @@ def lib():
         L.simint_hip_pairs_count.argtypes = [c_void_p]
         L.simint_hip_pairs_bytes.argtypes = [c_void_p]
         L.simint_hip_pairs_bytes.restype = c_size_t
-        L.simint_hip_compute_eri_prefix.argtypes = [c_void_p, c_void_p, c_int, c_int, iptr, llptr, c_double, c_void_p]
+        L.simint_hip_compute_eri_prefix.argtypes = [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_double,
+                                                    c_void_p]
         L.simint_hip_compute_eri_prefix.restype = ctypes.c_longlong
         L.simint_hip_compute_eri_diag.argtypes = [c_void_p, c_void_p]
         L.simint_hip_compute_eri_diag.restype = ctypes.c_longlong
@@ -113,11 +114,11 @@ def lib():
         L.simint_hip_compute_eri_list.argtypes = [c_void_p, c_void_p, ll, c_void_p, c_void_p, c_void_p, c_double,
                                                   c_void_p]
         L.simint_hip_compute_eri_list.restype = ll
-        L.simint_hip_compute_eri_range.argtypes = [c_void_p, c_void_p, c_int, c_int, iptr, iptr, llptr, c_double,
-                                                   c_int, c_void_p]
+        L.simint_hip_compute_eri_range.argtypes = [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p,
+                                                   c_double, c_int, c_void_p]
         L.simint_hip_compute_eri_range.restype = ll
-        L.simint_hip_compute_eri_deriv1_range.argtypes = [c_void_p, c_void_p, c_int, c_int, iptr, iptr, c_double,
-                                                          c_void_p, c_void_p]
+        L.simint_hip_compute_eri_deriv1_range.argtypes = [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p,
+                                                          c_double, c_void_p, c_void_p]
         L.simint_hip_compute_eri_deriv1_range.restype = ll
         L.simint_hip_deriv1_worksize.argtypes = [c_void_p, c_void_p, ll]
         L.simint_hip_deriv1_worksize.restype = ll
@@ -149,8 +150,8 @@ def lib():
         L.simint_hip_screen_counts.argtypes = [c_int, c_void_p, c_int, c_void_p, c_int, c_double, c_void_p]
         L.simint_hip_pairs_export.argtypes = [c_void_p, dptr, iptr, dptr]
         L.simint_hip_pairs_export.restype = ll
-        L.simint_hip_compute_jk_range.argtypes = [c_void_p, c_void_p, c_int, c_int, iptr, iptr, llptr, c_double,
-                                                  c_int, c_void_p, ctypes.POINTER(JK)]
+        L.simint_hip_compute_jk_range.argtypes = [c_void_p, c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p,
+                                                  c_double, c_int, c_void_p, ctypes.POINTER(JK)]
         L.simint_hip_compute_jk_range.restype = ll
         L.simint_hip_jk_symmetrize.argtypes = [c_int, c_void_p, c_void_p]
         L.simint_hip_shells_free.argtypes = [c_void_p]
@@ -444,8 +445,8 @@ def compute_range(P, Q, b0, ket_lo, ket_hi, out_off, d_out_ptr, screen_tol=0.0, 
     lo = None if ket_lo is None else np.ascontiguousarray(ket_lo, dtype=np.int32)
     out_off = np.ascontiguousarray(out_off, dtype=np.int64)
     r = lib().simint_hip_compute_eri_range(P.h, Q.h, int(b0), len(ket_hi),
-                                           None if lo is None else lo.ctypes.data_as(iptr),
-                                           ket_hi.ctypes.data_as(iptr), out_off.ctypes.data_as(llptr),
+                                           None if lo is None else lo.ctypes.data,
+                                           ket_hi.ctypes.data, out_off.ctypes.data,
                                            float(screen_tol), int(precision), c_void_p(d_out_ptr))
     if r < 0:
         raise RuntimeError("simint_hip_compute_eri_range failed (%d): %s" % (r, last_error()))
@@ -465,8 +466,8 @@ def compute_jk_range(P, Q, b0, ket_lo, ket_hi, out_off, d_out_ptr, jk, screen_to
     lo = None if ket_lo is None else np.ascontiguousarray(ket_lo, dtype=np.int32)
     out_off = np.ascontiguousarray(out_off, dtype=np.int64)
     r = lib().simint_hip_compute_jk_range(P.h, Q.h, int(b0), len(ket_hi),
-                                          None if lo is None else lo.ctypes.data_as(iptr),
-                                          ket_hi.ctypes.data_as(iptr), out_off.ctypes.data_as(llptr),
+                                          None if lo is None else lo.ctypes.data,
+                                          ket_hi.ctypes.data, out_off.ctypes.data,
                                           float(screen_tol), int(precision), c_void_p(d_out_ptr), ctypes.byref(jk))
     if r < 0:
         raise RuntimeError("simint_hip_compute_jk_range failed (%d): %s" % (r, last_error()))
@@ -484,8 +485,8 @@ def compute_deriv1_range(P, Q, b0, ket_lo, ket_hi, d_work, d_out_ptr, screen_tol
     ket_hi = np.ascontiguousarray(ket_hi, dtype=np.int32)
     lo = None if ket_lo is None else np.ascontiguousarray(ket_lo, dtype=np.int32)
     r = lib().simint_hip_compute_eri_deriv1_range(P.h, Q.h, int(b0), len(ket_hi),
-                                                  None if lo is None else lo.ctypes.data_as(iptr),
-                                                  ket_hi.ctypes.data_as(iptr), float(screen_tol),
+                                                  None if lo is None else lo.ctypes.data,
+                                                  ket_hi.ctypes.data, float(screen_tol),
                                                   c_void_p(d_work), c_void_p(d_out_ptr))
     if r < 0:
         raise RuntimeError("simint_hip_compute_eri_deriv1_range failed (%d): %s" % (r, last_error()))
@@ -495,8 +496,8 @@ def compute_deriv1_range(P, Q, b0, ket_lo, ket_hi, d_work, d_out_ptr, screen_tol
 def compute_prefix(P, Q, b0, nket, out_off, d_out_ptr, screen_tol=0.0):
     nket = np.ascontiguousarray(nket, dtype=np.int32)
     out_off = np.ascontiguousarray(out_off, dtype=np.int64)
-    r = lib().simint_hip_compute_eri_prefix(P.h, Q.h, int(b0), len(nket), nket.ctypes.data_as(iptr),
-                                            out_off.ctypes.data_as(llptr), float(screen_tol), c_void_p(d_out_ptr))
+    r = lib().simint_hip_compute_eri_prefix(P.h, Q.h, int(b0), len(nket), nket.ctypes.data,
+                                            out_off.ctypes.data, float(screen_tol), c_void_p(d_out_ptr))
     if r < 0:
         raise RuntimeError("simint_hip_compute_eri_prefix failed (%d): %s" % (r, last_error()))
     return r
