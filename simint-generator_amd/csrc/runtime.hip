@@ -17,6 +17,8 @@
 #include <stdlib.h>
 #include <string.h>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "simint/simint.h"
@@ -259,6 +261,9 @@ struct ThreadCtx {
     DevBuf in, out, items;
     DevBuf split;      // staging of the split lane-per-quartet kernels
     PinBuf stage;
+    PinBuf back;                    // results on their way to a caller's buffer
+    static constexpr int kSlots = 4;
+    hipEvent_t back_ev[kSlots] = {};     // per slot of it: the copy into it is done
     // Range launches queue without waiting for the ones before: on one
     // stream their device buffers (items, split) are reused in order.
     PinRing ring;
@@ -320,6 +325,107 @@ ThreadCtx &ctx()
     thread_local ThreadCtx *c = nullptr;
     if (!c) c = new ThreadCtx();
     return *c;
+}
+
+// ------------------------------------------- host buffers of the drop-in calls
+constexpr size_t kKernelCopy = 1 << 20;   // bytes up to which a kernel does the copy
+constexpr size_t kBackChunk = 4 << 20;    // bytes of one piece on the way back
+constexpr int kBackSlots = ThreadCtx::kSlots;
+constexpr int kBackThreads = 5;           // beside the calling thread
+
+__global__ void __launch_bounds__(256) copy_words(const double *__restrict__ from, double *__restrict__ to, size_t n)
+{
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) to[i] = from[i];
+}
+
+hipError_t launch_copy_words(const void *from, void *to, size_t words, hipStream_t s)
+{
+    const size_t nb = std::min<size_t>((words + 255) / 256, 256);
+    hipLaunchKernelGGL(copy_words, dim3((unsigned)nb), dim3(256), 0, s, static_cast<const double *>(from),
+                       static_cast<double *>(to), words);
+    return hipGetLastError();
+}
+
+// the first `bytes` of c.stage into c.in (both hold at least 1 MiB).  A
+// kernel that reads the pinned memory starts sooner than a copy command and
+// needs no hand-over between engines before the next kernel.
+hipError_t copy_in(ThreadCtx &c, size_t bytes)
+{
+    if (bytes <= kKernelCopy) return launch_copy_words(c.stage.p, c.in.p, (bytes + 7) / 8, c.s);
+    return hipMemcpyAsync(c.in.p, c.stage.p, bytes, hipMemcpyHostToDevice, c.s);
+}
+
+// n doubles from the device into the caller's pageable buffer, after the work
+// queued on c.s; done when it returns.  Small results are written to pinned
+// memory by a kernel.  Large ones come in pieces through a ring of pinned
+// slots, each divided among a few threads on its way into the caller's
+// buffer while the next ones cross PCIe: one thread's memcpy (what a copy
+// command to pageable memory does) is several times slower than the link.
+hipError_t copy_back(ThreadCtx &c, double *dst, const double *src, size_t n)
+{
+    hipError_t e;
+    const size_t bytes = sizeof(double) * n;
+    if ((e = c.back.reserve(bytes <= kKernelCopy ? bytes : kBackSlots * kBackChunk)) != hipSuccess) return e;
+    char *pin = static_cast<char *>(c.back.p);
+    if (bytes <= kKernelCopy) {
+        if ((e = launch_copy_words(src, pin, n, c.s)) != hipSuccess) return e;
+        if ((e = hipStreamSynchronize(c.s)) != hipSuccess) return e;
+        memcpy(dst, pin, bytes);
+        return hipSuccess;
+    }
+    for (hipEvent_t &ev : c.back_ev)
+        if (!ev && (e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return e;
+    const long long npiece = (long long)((bytes + kBackChunk - 1) / kBackChunk);
+    auto piece_bytes = [&](long long k) { return std::min(kBackChunk, bytes - (size_t)k * kBackChunk); };
+    auto queue = [&](long long k) {
+        const hipError_t r = hipMemcpyAsync(pin + (size_t)(k % kBackSlots) * kBackChunk,
+                                            reinterpret_cast<const char *>(src) + (size_t)k * kBackChunk,
+                                            piece_bytes(k), hipMemcpyDeviceToHost, c.s);
+        return r != hipSuccess ? r : hipEventRecord(c.back_ev[k % kBackSlots], c.s);
+    };
+    std::atomic<long long> ready{0};                       // pieces that have arrived (-1: give up)
+    std::atomic<long long> copied[kBackThreads] = {};      // pieces each thread is done with
+    int nthread = 0;
+    auto part = [&](long long k, int t) {                  // thread t's part of piece k
+        const size_t m = piece_bytes(k), p = (m / (nthread + 1) + 63) & ~(size_t)63;
+        const size_t lo = std::min(m, p * t), hi = t == nthread ? m : std::min(m, p * (t + 1));
+        memcpy(reinterpret_cast<char *>(dst) + (size_t)k * kBackChunk + lo,
+               pin + (size_t)(k % kBackSlots) * kBackChunk + lo, hi - lo);
+    };
+    std::atomic<int> go{0};
+    auto helper = [&](int t) {
+        while (!go.load(std::memory_order_acquire)) std::this_thread::yield();
+        for (long long k = 0; k < npiece; k++) {
+            long long r;
+            while ((r = ready.load(std::memory_order_acquire)) >= 0 && r <= k) std::this_thread::yield();
+            if (r < 0) return;
+            part(k, t);
+            copied[t].store(k + 1, std::memory_order_release);
+        }
+    };
+    std::thread helpers[kBackThreads];
+    try {
+        const int most = std::min<int>(kBackThreads, (int)std::thread::hardware_concurrency() / 2);
+        for (; nthread < most; nthread++) helpers[nthread] = std::thread(helper, nthread);
+    } catch (const std::system_error &) {
+        // as many as could be started
+    }
+    go.store(1, std::memory_order_release);
+    e = hipSuccess;
+    for (long long k = 0; k < std::min<long long>(kBackSlots, npiece) && e == hipSuccess; k++) e = queue(k);
+    for (long long k = 0; k < npiece && e == hipSuccess; k++) {
+        if ((e = hipEventSynchronize(c.back_ev[k % kBackSlots])) != hipSuccess) break;
+        ready.store(k + 1, std::memory_order_release);
+        part(k, nthread);
+        if (k + kBackSlots < npiece) {
+            for (int t = 0; t < nthread; t++)
+                while (copied[t].load(std::memory_order_acquire) <= k) std::this_thread::yield();
+            e = queue(k + kBackSlots);
+        }
+    }
+    if (e != hipSuccess) ready.store(-1, std::memory_order_release);
+    for (int t = 0; t < nthread; t++) helpers[t].join();
+    return e;
 }
 
 // ---------------------------------------------------------------- packing
@@ -855,8 +961,8 @@ int simint_compute_ostei_deriv(int deriv, const simint_multi_shellpair *P, const
     hipError_t e;
     // an earlier asynchronous call of this thread (_range, _prefix, _diag)
     // may still read c.stage or c.split: wait for it before reuse
-    if ((e = c.range_enter()) != hipSuccess) { set_err("hipStreamWaitEvent", e); return SIMINT_ERROR_HIP; }
     if ((e = hipStreamSynchronize(c.s)) != hipSuccess) { set_err("hipStreamSynchronize", e); return SIMINT_ERROR_HIP; }
+    if ((e = c.range_enter()) != hipSuccess) { set_err("hipStreamWaitEvent", e); return SIMINT_ERROR_HIP; }
     const size_t final_n = (size_t)nP * nQ * nc * (deriv ? 12 : 1);
     const bool gamess = gamess_needed(am);
     const size_t out_bytes = sizeof(double) * (scratch + (deriv ? final_n : 0) + (gamess ? final_n : 0));
@@ -864,8 +970,7 @@ int simint_compute_ostei_deriv(int deriv, const simint_multi_shellpair *P, const
     if ((e = c.in.reserve(im.buf.size())) != hipSuccess) { set_err("hipMalloc", e); return SIMINT_ERROR_HIP; }
     if ((e = c.out.reserve(out_bytes)) != hipSuccess) { set_err("hipMalloc", e); return SIMINT_ERROR_HIP; }
     memcpy(c.stage.p, im.buf.data(), im.buf.size());
-    e = hipMemcpyAsync(c.in.p, c.stage.p, im.buf.size(), hipMemcpyHostToDevice, c.s);
-    if (e != hipSuccess) { set_err("hipMemcpyAsync(H2D)", e); return SIMINT_ERROR_HIP; }
+    if ((e = copy_in(c, im.buf.size())) != hipSuccess) { set_err("copy to the device", e); return SIMINT_ERROR_HIP; }
 
     size_t nst = 0;
     for (auto &t : terms) nst = std::max(nst, (size_t)simint_dispatch_staging(t.am[0], t.am[1], t.am[2], t.am[3]));
@@ -930,14 +1035,11 @@ int simint_compute_ostei_deriv(int deriv, const simint_multi_shellpair *P, const
         }
         result = perm;
     }
-    e = hipMemcpyAsync(integrals, result, sizeof(double) * final_n, hipMemcpyDeviceToHost, c.s);
-    if (e != hipSuccess) {
-        set_err("hipMemcpyAsync(D2H)", e);
+    if ((e = copy_back(c, integrals, result, final_n)) != hipSuccess) {
+        set_err("copy from the device", e);
         hipStreamSynchronize(c.s);
         return SIMINT_ERROR_HIP;
     }
-    e = hipStreamSynchronize(c.s);
-    if (e != hipSuccess) { set_err("hipStreamSynchronize", e); return SIMINT_ERROR_HIP; }
     return nP * nQ;
 }
 
@@ -1242,8 +1344,8 @@ long long simint_hip_compute_eri_diag(const simint_hip_pairs *P, double *d_out)
         items[b].obase = 0;
     }
     hipError_t e;
-    if ((e = c.range_enter()) != hipSuccess) { set_err("hipStreamWaitEvent", e); return SIMINT_ERROR_HIP; }
     if ((e = hipStreamSynchronize(c.s)) != hipSuccess) { set_err("hipStreamSynchronize", e); return SIMINT_ERROR_HIP; }
+    if ((e = c.range_enter()) != hipSuccess) { set_err("hipStreamWaitEvent", e); return SIMINT_ERROR_HIP; }
     const size_t bytes = sizeof(WorkItem) * items.size();
     if ((e = c.stage.reserve(bytes)) != hipSuccess) { set_err("hipHostMalloc", e); return SIMINT_ERROR_HIP; }
     if ((e = c.items.reserve(bytes)) != hipSuccess) { set_err("hipMalloc", e); return SIMINT_ERROR_HIP; }

@@ -1,10 +1,14 @@
-"""Range launches queued one behind another.
+"""Range launches queued one behind another, and results on their way into a
+caller's buffer.
 
 Range launches describe their ranges in a ring of pinned memory (two halves
 of 1 MiB) and share the thread's item and staging buffers: many launches of
 changing ranges are queued without a wait, past both ends of the ring, over
 a change of stream, and compared bit for bit with the same launches waited
-for one by one."""
+for one by one.  A host-buffer call copies its results back in one kernel up
+to 1 MiB and in 4 MiB pieces through four slots above: sizes at both edges,
+one piece, a ragged last piece and more pieces than slots, against the
+device-resident integrals of the same kernel."""
 import ctypes
 
 import numpy as np
@@ -98,4 +102,27 @@ def test_range_refused_under_capture(gpu):
     simint.synchronize()
     assert torch.equal(out, want)
     for h in (P, hp, b):
+        h.free()
+
+
+# values: 9, 131058, 131130 (1 MiB is 131072), 524286 and 524295 (4 MiB is
+# 524288), six pieces, and sixteen and a bit
+@pytest.mark.parametrize("nbra,nket", [(1, 1), (3, 4854), (2, 7285), (6, 9709), (5, 11651), (45, 7767), (77, 12107)])
+def test_results_to_the_host(gpu, nbra, nket):
+    rng = np.random.default_rng(nbra)
+    bb, hp, P = _pairs(rng, (1, 0), nbra, depth=1)
+    bk, hq, Q = _pairs(rng, (1, 0), nket, depth=1)
+    nv = 9 * nbra * nket
+    dev = torch.full((nv,), float("nan"), dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    simint.compute_range(P, Q, 0, None, np.full(nbra, nket, dtype=np.int32),
+                         9 * nket * np.arange(nbra, dtype=np.int64), dev.data_ptr())
+    simint.synchronize()
+    got = np.full(nv + 1, np.nan)
+    rc = simint.lib().simint_compute_eri(ctypes.byref(hp.mp), ctypes.byref(hq.mp), 0.0, None,
+                                         got.ctypes.data_as(simint.dptr))
+    assert rc == nbra * nket
+    assert np.isnan(got[-1])
+    assert np.array_equal(got[:-1], dev.cpu().numpy())
+    for h in (P, Q, hp, hq, bb, bk):
         h.free()
