@@ -1522,6 +1522,7 @@ long long deriv1_list(const simint_hip_pairs *P, const simint_hip_pairs *Q, long
         }
         a.out = d_work + t.off * nquartet;
         a.ostride = t.nc;
+        a.split = list_split(nquartet);
         if ((e = fns[k](&a, c.s)) != hipSuccess) { set_err("class kernel launch", e); return SIMINT_ERROR_HIP; }
         if (t.sign > 0) d.plus[t.centre] = a.out;
         else d.minus[t.centre] = a.out;
