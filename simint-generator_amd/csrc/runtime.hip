@@ -275,6 +275,25 @@ struct ThreadCtx {
     {
         hipStreamCreateWithFlags(&own, hipStreamNonBlocking);
         s = own;
+        // now, not when first needed: streams are dealt out over the few
+        // hardware queues in the order of their creation, and these are to
+        // have other queues than own
+        make_side();
+    }
+    // side streams for the terms of one derivative range
+    static constexpr int kSide = 3;
+    hipStream_t side[kSide] = {};
+    hipEvent_t fork_ev = nullptr, join_ev[kSide] = {};
+    hipError_t make_side()
+    {
+        if (fork_ev) return hipSuccess;
+        hipError_t e;
+        for (int k = 0; k < kSide; k++) {
+            if (!side[k] && (e = hipStreamCreateWithFlags(&side[k], hipStreamNonBlocking)) != hipSuccess) return e;
+            if (!join_ev[k] && (e = hipEventCreateWithFlags(&join_ev[k], hipEventDisableTiming)) != hipSuccess)
+                return e;
+        }
+        return hipEventCreateWithFlags(&fork_ev, hipEventDisableTiming);
     }
     // before s is left, or its work is captured: the range work queued on it
     // ends at range_ev
@@ -1112,6 +1131,9 @@ namespace {
 
 constexpr int kMaxTerms = 8;
 constexpr int kExpandLanes = 8;   // threads per bra
+// Work items up to which the terms of a derivative run side by side: eight
+// wavefronts a compute unit.  More fill the chip by themselves.
+constexpr long long kForkItems = 2048;
 
 // What a range launch covers, in pinned host memory: per bra its ket range,
 // its first item and, per term, its output offset.
@@ -1250,7 +1272,34 @@ long long range_launch(const simint_hip_pairs *P, const simint_hip_pairs *Q, int
     const unsigned nblk = (unsigned)((n * kExpandLanes + 255) / 256);
     hipLaunchKernelGGL(expand_range_items, dim3(nblk, nterm), dim3(256), 0, c.s, x);
     if ((e = hipGetLastError()) != hipSuccess) { set_err("expand launch", e); return SIMINT_ERROR_HIP; }
-    for (int t = 0; t < nterm; t++) {
+    // stream of each term: 0 is c.s, k > 0 side stream k - 1
+    int on[kMaxTerms] = {};
+    bool used[ThreadCtx::kSide + 1] = {};
+    if (nterm > 1 && nitems <= kForkItems) {
+        double load[ThreadCtx::kSide + 1] = {};
+        int order[kMaxTerms];
+        double cost[kMaxTerms];
+        for (int t = 0; t < nterm; t++) {
+            const int l = terms[t].am[0] + terms[t].am[1] + terms[t].am[2] + terms[t].am[3];
+            cost[t] = (double)x.stride[t] * (l + 1) * (l + 1);
+            order[t] = t;
+        }
+        std::sort(order, order + nterm, [&](int a, int b) { return cost[a] > cost[b]; });
+        for (int k = 0; k < nterm; k++) {
+            const RangeTerm &T = terms[order[k]];
+            // kernels that stage share c.split: one after another
+            if (!simint_dispatch_staging(T.am[0], T.am[1], T.am[2], T.am[3]))
+                on[order[k]] = (int)(std::min_element(load, load + ThreadCtx::kSide + 1) - load);
+            load[on[order[k]]] += cost[order[k]];
+            used[on[order[k]]] = true;
+        }
+        if ((e = c.make_side()) == hipSuccess) e = hipEventRecord(c.fork_ev, c.s);
+        for (int k = 0; k < ThreadCtx::kSide && e == hipSuccess; k++)
+            if (used[k + 1]) e = hipStreamWaitEvent(c.side[k], c.fork_ev, 0);
+        if (e != hipSuccess) { set_err("side streams", e); return SIMINT_ERROR_HIP; }
+    }
+    hipError_t failed = hipSuccess;
+    for (int t = 0; t < nterm && failed == hipSuccess; t++) {
         const RangeTerm &T = terms[t];
         EriArgs a;
         a.scratch = static_cast<double *>(c.split.p);
@@ -1267,8 +1316,17 @@ long long range_launch(const simint_hip_pairs *P, const simint_hip_pairs *Q, int
         a.tol2 = (screen_tol > 0.0 && P->has_screen && Q->has_screen) ? screen_tol * screen_tol : 0.0;
         a.ket_screen_max = Q->screen_max;
         a.stride = x.stride[t];
-        if ((e = T.fn(&a, c.s)) != hipSuccess) { set_err("class kernel launch", e); return SIMINT_ERROR_HIP; }
+        failed = T.fn(&a, on[t] ? c.side[on[t] - 1] : c.s);
     }
+    for (int k = 0; k < ThreadCtx::kSide; k++) {
+        if (!used[k + 1]) continue;
+        if ((e = hipEventRecord(c.join_ev[k], c.side[k])) == hipSuccess) e = hipStreamWaitEvent(c.s, c.join_ev[k], 0);
+        if (e != hipSuccess) {   // nothing of the call may run on beside what is queued after it
+            hipStreamSynchronize(c.side[k]);
+            if (failed == hipSuccess) failed = e;
+        }
+    }
+    if (failed != hipSuccess) { set_err("class kernel launch", failed); return SIMINT_ERROR_HIP; }
     if (items_out) *items_out = x.items;
     if (nitems_out) *nitems_out = nitems;
     if (tstart_out) *tstart_out = x.tstart;
