@@ -24,6 +24,7 @@
 // (jk_digest_rows).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 
 #include "simint/simint_eri.h"
@@ -139,18 +140,13 @@ __global__ void __launch_bounds__(256) jk_digest(const WorkItem *items, long lon
 // per row), instead of one pass over the quartet per update.  The second
 // ket shell's components are taken DC at a time (DC divides ND, chosen so
 // the accumulators stay in registers), each chunk reading its columns of
-// every row.  rows != nullptr (ROWS): the exchange updates whose row is a
-// bra function (K_a., K_b.) go to that block's row accumulator in the local
-// data share -- row a of the first bra shell at rows[a * nbf], row b of the
-// second at rows[(na + b) * nbf] -- and K_b. is added there after every
-// row (a, b); without it they go to global memory, K_b. summed over a first.
-template <int NB, int NC, int ND, int DC, bool ROWS>
+// every row.  K_b. is summed over a before it goes to global memory.
+template <int NB, int NC, int ND, int DC>
 __device__ __forceinline__ void digest_item(const WorkItem &it, int lane, const long long *col, const double *ints,
-                                            int na, const JkDev &jk, double *rows)
+                                            int na, const JkDev &jk)
 {
     static_assert(ND % DC == 0, "chunks of the second ket shell divide it");
     constexpr int NCD = NC * ND;
-    constexpr int KB = ROWS ? 1 : NB;   // K_b. accumulators held across a
     const int n = jk.nbf;
     const int fa = jk.bra_fun[2 * it.bra], fb = jk.bra_fun[2 * it.bra + 1];
     if (fa < 0 || fb < 0 || fa + na > n || fb + NB > n) return;
@@ -169,15 +165,9 @@ __device__ __forceinline__ void digest_item(const WorkItem &it, int lane, const 
     const double *q = ints + it.obase + kq * (long long)(na * NB * NCD);
     const double *__restrict__ D = jk.D;
     auto Dl = [&](long long idx) { return D[act ? idx : 0]; };
-    // exchange row update: row r of the bra's (na + NB) rows, column c
+    // exchange update: row r of the bra's (na + NB) rows, column c
     auto addK = [&](int r, int c, double v) {
-        if constexpr (ROWS) {
-            // the local data share, named as such so the add is a ds_add_f64
-            __attribute__((address_space(3))) double *lds = (__attribute__((address_space(3))) double *)rows;
-            atomicAdd((double *)(lds + (long long)r * n + c), v);
-        } else {
-            unsafeAtomicAdd(jk.K + (long long)(r < na ? fa + r : fb + r - na) * n + c, v);
-        }
+        unsafeAtomicAdd(jk.K + (long long)(r < na ? fa + r : fb + r - na) * n + c, v);
     };
     double f = act ? 1.0 : 0.0;
     if (fa == fb) f *= 0.5;
@@ -185,7 +175,7 @@ __device__ __forceinline__ void digest_item(const WorkItem &it, int lane, const 
     if (jk.same && k == it.bra) f *= 0.5;
     const double g = 2.0 * f;
     for (int d0 = 0; d0 < ND; d0 += DC) {
-        double dcd[NC * DC], jcd[NC * DC], kbc[KB][NC], kbd[KB][DC];
+        double dcd[NC * DC], jcd[NC * DC], kbc[NB][NC], kbd[NB][DC];
 #pragma unroll
         for (int c = 0; c < NC; c++)
 #pragma unroll
@@ -194,7 +184,7 @@ __device__ __forceinline__ void digest_item(const WorkItem &it, int lane, const 
                 jcd[c * DC + d] = 0.0;
             }
 #pragma unroll
-        for (int b = 0; b < KB; b++) {
+        for (int b = 0; b < NB; b++) {
 #pragma unroll
             for (int c = 0; c < NC; c++) kbc[b][c] = 0.0;
 #pragma unroll
@@ -214,13 +204,6 @@ __device__ __forceinline__ void digest_item(const WorkItem &it, int lane, const 
             }
             // one row (a, b, :, d0..d0+DC) of the quartet
             auto row = [&](int b) {
-                const int kb = ROWS ? 0 : b;
-                if constexpr (ROWS) {
-#pragma unroll
-                    for (int c = 0; c < NC; c++) kbc[0][c] = 0.0;
-#pragma unroll
-                    for (int d = 0; d < DC; d++) kbd[0][d] = 0.0;
-                }
                 double dbd[DC], dbc[NC];
 #pragma unroll
                 for (int d = 0; d < DC; d++) dbd[d] = Dl((long long)(fb + b) * n + fd + d0 + d);
@@ -238,30 +221,227 @@ __device__ __forceinline__ void digest_item(const WorkItem &it, int lane, const 
                         jcd[c * DC + d] = fma(v, dab, jcd[c * DC + d]);
                         kac[c] = fma(v, dbd[d], kac[c]);
                         kad[d] = fma(v, dbc[c], kad[d]);
-                        kbc[kb][c] = fma(v, dad[d], kbc[kb][c]);
-                        kbd[kb][d] = fma(v, dac[c], kbd[kb][d]);
+                        kbc[b][c] = fma(v, dad[d], kbc[b][c]);
+                        kbd[b][d] = fma(v, dac[c], kbd[b][d]);
                     }
                 if (jk.J) {
                     jab = wave_sum(f * jab);
                     if (lane == 0) unsafeAtomicAdd(jk.J + (long long)(fa + a) * n + fb + b, 4.0 * jab);
                 }
-                if constexpr (ROWS) {
-                    if (jk.K && act) {
+            };
 #pragma unroll
-                        for (int c = 0; c < NC; c++) addK(na + b, fc + c, g * kbc[0][c]);
+            for (int b = 0; b < NB; b++) row(b);
+            if (jk.K && act) {
 #pragma unroll
-                        for (int d = 0; d < DC; d++) addK(na + b, fd + d0 + d, g * kbd[0][d]);
+                for (int c = 0; c < NC; c++) addK(a, fc + c, g * kac[c]);
+#pragma unroll
+                for (int d = 0; d < DC; d++) addK(a, fd + d0 + d, g * kad[d]);
+            }
+        }
+        if (act && jk.J) {
+#pragma unroll
+            for (int c = 0; c < NC; c++)
+#pragma unroll
+                for (int d = 0; d < DC; d++)
+                    unsafeAtomicAdd(jk.J + (long long)(fc + c) * n + fd + d0 + d, 4.0 * f * jcd[c * DC + d]);
+        }
+        if (act && jk.K) {
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+#pragma unroll
+                for (int c = 0; c < NC; c++) addK(na + b, fc + c, g * kbc[b][c]);
+#pragma unroll
+                for (int d = 0; d < DC; d++) addK(na + b, fd + d0 + d, g * kbd[b][d]);
+            }
+        }
+    }
+}
+
+// one wavefront per work item
+template <int NB, int NC, int ND, int DC>
+__global__ void __launch_bounds__(256) jk_digest_t(const WorkItem *items, long long nitems, const long long *col,
+                                                   const double *ints, int na, JkDev jk)
+{
+    const long long w = (long long)blockIdx.x * 4 + threadIdx.x / 64;
+    if (w >= nitems) return;   // uniform over the wave
+    digest_item<NB, NC, ND, DC>(items[w], threadIdx.x & 63, col, ints, na, jk);
+}
+
+// Doubles a lane of the per-bra kernel holds beyond the ket block's density
+// and Coulomb sums when it keeps the second bra shell's exchange sums and
+// density rows over all a and the integrals of two a at a time (held(): all
+// loads of an a in flight together, each ket's cache lines read while they
+// are in the L1 cache, and a row of the exchange added to the local data
+// share once instead of na times).
+constexpr int kHeldDoubles = 108;
+constexpr bool held(int nb, int nc, int dc)
+{
+    return 2 * nc * dc + 4 * (nc + dc) + 2 * nb * (nc + dc) + 2 * nb * nc * dc <= kHeldDoubles;
+}
+
+// Where it cannot, the next row's integrals are loaded ahead if two rows fit.
+constexpr bool ahead(int nc, int dc) { return 4 * nc * dc + 4 * (nc + dc) <= 72; }
+
+// Most threads of the per-bra kernel's block: two wavefronts a SIMD have 256
+// registers each, which the f classes exceed.
+constexpr int rows_threads(int nb, int nc, int nd) { return nb > 6 || nc > 6 || nd > 6 ? 256 : 512; }
+
+// The per-bra kernel's work on one item: a in [a0, a1) of its quartets.  The
+// exchange rows of the bra's functions, rows[r * nbf] (r < na: first shell),
+// and the lanes' sums of J_ab, jsum[(a * NB + b) * 64 + lane], are in the
+// local data share: both adds are fire and forget, where a sum over the
+// wavefront for every (a, b) waited for twelve dependent exchanges.  Every
+// wait is for loads issued a step ahead: the next a's integrals (held) or
+// the next row's.
+template <int NB, int NC, int ND, int DC>
+__device__ __forceinline__ void digest_rows_item(const WorkItem &it, int lane, const long long *col,
+                                                 const double *ints, int na, int a0, int a1, const JkDev &jk,
+                                                 double *rows, double *jsum)
+{
+    static_assert(ND % DC == 0, "chunks of the second ket shell divide it");
+    constexpr int NCD = NC * ND, NV = NC * DC;
+    constexpr bool HOLD = held(NB, NC, DC), AHEAD = HOLD || ahead(NC, DC);
+    constexpr int KB = HOLD ? NB : 1;
+    constexpr int STEP = HOLD ? NB : 1;     // rows loaded at a time
+    const int n = jk.nbf;
+    const int fa = jk.bra_fun[2 * it.bra], fb = jk.bra_fun[2 * it.bra + 1];
+    if (fa < 0 || fb < 0 || fa + na > n || fb + NB > n) return;
+    bool act = lane >= it.lane_lo && lane < it.lane_hi;
+    const long long k = act ? col[(long long)it.tile * 64 + lane] : -1;
+    act = act && k >= 0;
+    int fc = 0, fd = 0;
+    if (act) {
+        fc = jk.ket_fun[2 * k];
+        fd = jk.ket_fun[2 * k + 1];
+        act = fc >= 0 && fd >= 0 && fc + NC <= n && fd + ND <= n;
+    }
+    // idle lanes read a quartet of the item (its first lane's, which the
+    // class kernel wrote) and density element 0, and add nothing
+    const long long kq = act ? k : col[(long long)it.tile * 64 + it.lane_lo];
+    const double *q = ints + it.obase + kq * (long long)(na * NB * NCD);
+    const double *__restrict__ D = jk.D;
+    auto Dl = [&](long long idx) { return D[act ? idx : 0]; };
+    auto ldsadd = [](double *p, double v) {
+        // the local data share, named as such so the add is a ds_add_f64
+        atomicAdd((double *)(__attribute__((address_space(3))) double *)p, v);
+    };
+    auto addK = [&](int r, int c, double v) { ldsadd(rows + (long long)r * n + c, v); };
+    double f = act ? 1.0 : 0.0;
+    if (fa == fb) f *= 0.5;
+    if (fc == fd) f *= 0.5;
+    if (jk.same && k == it.bra) f *= 0.5;
+    const double g = 2.0 * f;
+    for (int d0 = 0; d0 < ND; d0 += DC) {
+        double dcd[NV], jcd[NV], kbc[KB][NC], kbd[KB][DC], dbc[KB][NC], dbd[KB][DC];
+        double cur[STEP * NV], nxt[AHEAD ? STEP * NV : 1];
+        // rows r .. r + STEP of the quartet, columns of this chunk
+        auto load = [&](double *v, int r) {
+            const double *p = q + (long long)r * NCD + d0;
+#pragma unroll
+            for (int s = 0; s < STEP; s++)
+#pragma unroll
+                for (int c = 0; c < NC; c++)
+#pragma unroll
+                    for (int d = 0; d < DC; d++) v[s * NV + c * DC + d] = p[s * NCD + c * ND + d];
+        };
+        auto load_db = [&](int kb, int b) {
+#pragma unroll
+            for (int c = 0; c < NC; c++) dbc[kb][c] = Dl((long long)(fb + b) * n + fc + c);
+#pragma unroll
+            for (int d = 0; d < DC; d++) dbd[kb][d] = Dl((long long)(fb + b) * n + fd + d0 + d);
+        };
+        auto clear_kb = [&](int kb) {
+#pragma unroll
+            for (int c = 0; c < NC; c++) kbc[kb][c] = 0.0;
+#pragma unroll
+            for (int d = 0; d < DC; d++) kbd[kb][d] = 0.0;
+        };
+        auto add_kb = [&](int kb, int b) {
+            if (!jk.K || !act) return;
+#pragma unroll
+            for (int c = 0; c < NC; c++) addK(na + b, fc + c, g * kbc[kb][c]);
+#pragma unroll
+            for (int d = 0; d < DC; d++) addK(na + b, fd + d0 + d, g * kbd[kb][d]);
+        };
+        if constexpr (AHEAD) load(cur, a0 * NB);
+#pragma unroll
+        for (int c = 0; c < NC; c++)
+#pragma unroll
+            for (int d = 0; d < DC; d++) {
+                dcd[c * DC + d] = Dl((long long)(fc + c) * n + fd + d0 + d);
+                jcd[c * DC + d] = 0.0;
+            }
+        if constexpr (HOLD) {
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                load_db(b, b);
+                clear_kb(b);
+            }
+        }
+        for (int a = a0; a < a1; a++) {
+            double dad[DC], dac[NC], kac[NC], kad[DC];
+            if constexpr (HOLD) {
+                if (a + 1 < a1) load(nxt, (a + 1) * NB);
+            }
+#pragma unroll
+            for (int d = 0; d < DC; d++) {
+                dad[d] = Dl((long long)(fa + a) * n + fd + d0 + d);
+                kad[d] = 0.0;
+            }
+#pragma unroll
+            for (int c = 0; c < NC; c++) {
+                dac[c] = Dl((long long)(fa + a) * n + fc + c);
+                kac[c] = 0.0;
+            }
+            // row (a, b) of the quartet, its values at v
+            auto row = [&](int b, int kb, const double *v) {
+                const double dab = D[(long long)(fa + a) * n + fb + b];
+                double jab = 0.0;
+#pragma unroll
+                for (int c = 0; c < NC; c++)
+#pragma unroll
+                    for (int d = 0; d < DC; d++) {
+                        const double x = act ? v[c * DC + d] : 0.0;
+                        jab = fma(x, dcd[c * DC + d], jab);
+                        jcd[c * DC + d] = fma(x, dab, jcd[c * DC + d]);
+                        kac[c] = fma(x, dbd[kb][d], kac[c]);
+                        kad[d] = fma(x, dbc[kb][c], kad[d]);
+                        kbc[kb][c] = fma(x, dad[d], kbc[kb][c]);
+                        kbd[kb][d] = fma(x, dac[c], kbd[kb][d]);
+                    }
+                if (jk.J) {
+                    if (jsum) {
+                        ldsadd(jsum + (a * NB + b) * 64 + lane, f * jab);
+                    } else {
+                        jab = wave_sum(f * jab);
+                        if (lane == 0) unsafeAtomicAdd(jk.J + (long long)(fa + a) * n + fb + b, 4.0 * jab);
                     }
                 }
             };
-            if constexpr (ROWS) {
-                // nothing is indexed by b: a loop, so one row's loads are in
-                // flight at a time
-#pragma unroll 1
-                for (int b = 0; b < NB; b++) row(b);
-            } else {
+            if constexpr (HOLD) {
 #pragma unroll
-                for (int b = 0; b < NB; b++) row(b);
+                for (int b = 0; b < NB; b++) row(b, b, cur + b * NV);
+#pragma unroll
+                for (int i = 0; i < STEP * NV; i++) cur[i] = nxt[i];
+            } else {
+                // nothing is indexed by b: a loop, at most one row's loads ahead
+#pragma unroll 1
+                for (int b = 0; b < NB; b++) {
+                    load_db(0, b);
+                    clear_kb(0);
+                    const int r = a * NB + b;
+                    if constexpr (AHEAD) {
+                        if (r + 1 < a1 * NB) load(nxt, r + 1);
+                    } else {
+                        load(cur, r);
+                    }
+                    row(b, 0, cur);
+                    add_kb(0, b);
+                    if constexpr (AHEAD) {
+#pragma unroll
+                        for (int i = 0; i < NV; i++) cur[i] = nxt[i];
+                    }
+                }
             }
             if (jk.K && act) {
 #pragma unroll
@@ -277,41 +457,25 @@ __device__ __forceinline__ void digest_item(const WorkItem &it, int lane, const 
                 for (int d = 0; d < DC; d++)
                     unsafeAtomicAdd(jk.J + (long long)(fc + c) * n + fd + d0 + d, 4.0 * f * jcd[c * DC + d]);
         }
-        if constexpr (!ROWS) {
-            if (act && jk.K) {
+        if constexpr (HOLD) {
 #pragma unroll
-                for (int b = 0; b < NB; b++) {
-#pragma unroll
-                    for (int c = 0; c < NC; c++) addK(na + b, fc + c, g * kbc[b][c]);
-#pragma unroll
-                    for (int d = 0; d < DC; d++) addK(na + b, fd + d0 + d, g * kbd[b][d]);
-                }
-            }
+            for (int b = 0; b < NB; b++) add_kb(b, b);
         }
     }
 }
 
-// one wavefront per work item
+// One block per bra pair of the launch: its wavefronts take the bra's work
+// items (or, where the launch has few, parts of their a) in turn,
+// and the exchange rows of the bra's functions and J_ab are summed over all
+// its kets in the local data share ((na + NB) x nbf and na x NB x 64
+// doubles, dynamic) and added to K and J once per touched element at the
+// end -- never more global atomics than one per quartet and element, usually
+// far fewer (every ket of the bra adds to the same rows).  Launched only
+// with an exchange matrix to fill.
 template <int NB, int NC, int ND, int DC>
-__global__ void __launch_bounds__(256) jk_digest_t(const WorkItem *items, long long nitems, const long long *col,
-                                                   const double *ints, int na, JkDev jk)
-{
-    const long long w = (long long)blockIdx.x * 4 + threadIdx.x / 64;
-    if (w >= nitems) return;   // uniform over the wave
-    digest_item<NB, NC, ND, DC, false>(items[w], threadIdx.x & 63, col, ints, na, jk, nullptr);
-}
-
-// One block per bra pair of the launch: its four wavefronts take the bra's
-// work items in turn, and the exchange rows of the bra's functions are
-// summed over all its kets in the local data share ((na + NB) x nbf
-// doubles, dynamic) and added to K once per touched element at the end --
-// never more global atomics than one per quartet and element, usually far
-// fewer (every ket of the bra adds to the same rows).  Launched only with
-// an exchange matrix to fill.
-template <int NB, int NC, int ND, int DC>
-__global__ void __launch_bounds__(256) jk_digest_rows(const WorkItem *items, long long nitems,
+__global__ void __launch_bounds__(rows_threads(NB, NC, ND)) jk_digest_rows(const WorkItem *items, long long nitems,
                                                       const long long *tstart, int nbra, const long long *col,
-                                                      const double *ints, int na, JkDev jk)
+                                                      const double *ints, int na, int parts, int lanesum, JkDev jk)
 {
     extern __shared__ double rows[];
     const int bi = blockIdx.x;
@@ -319,20 +483,30 @@ __global__ void __launch_bounds__(256) jk_digest_rows(const WorkItem *items, lon
     if (i0 >= i1) return;   // uniform over the block
     const int n = jk.nbf;
     const int R = na + NB;
-    for (long long e = threadIdx.x; e < (long long)R * n; e += 256) rows[e] = 0.0;
+    double *jsum = lanesum ? rows + R * n : nullptr;
+    const int nlds = R * n + (lanesum ? na * NB * 64 : 0);   // at most 160 KB
+    for (int e = threadIdx.x; e < nlds; e += blockDim.x) rows[e] = 0.0;
     __syncthreads();
-    const int lane = threadIdx.x & 63;
-    for (long long w = i0 + threadIdx.x / 64; w < i1; w += 4)
-        digest_item<NB, NC, ND, DC, true>(items[w], lane, col, ints, na, jk, rows);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x / 64, nwave = blockDim.x / 64;
+    for (int u = wave; u < (int)(i1 - i0) * parts; u += nwave) {
+        const int w = u / parts, p = u - w * parts;
+        digest_rows_item<NB, NC, ND, DC>(items[i0 + w], lane, col, ints, na, p * na / parts, (p + 1) * na / parts,
+                                         jk, rows, jsum);
+    }
     __syncthreads();
     const int bra = items[i0].bra;
     const int fa = jk.bra_fun[2 * bra], fb = jk.bra_fun[2 * bra + 1];
     if (fa < 0 || fb < 0 || fa + na > n || fb + NB > n) return;
-    for (long long e = threadIdx.x; e < (long long)R * n; e += 256) {
+    for (int e = threadIdx.x; e < R * n; e += blockDim.x) {
         const double v = rows[e];
         if (v == 0.0) continue;
-        const int r = (int)(e / n), c = (int)(e - (long long)r * n);
+        const int r = e / n, c = e - r * n;
         unsafeAtomicAdd(jk.K + (long long)(r < na ? fa + r : fb + r - na) * n + c, v);
+    }
+    if (!jk.J || !jsum) return;
+    for (int r = wave; r < na * NB; r += nwave) {
+        const double s = wave_sum(jsum[r * 64 + lane]);
+        if (lane == 0) unsafeAtomicAdd(jk.J + (long long)(fa + r / NB) * n + fb + r % NB, 4.0 * s);
     }
 }
 
@@ -364,6 +538,10 @@ constexpr int pick_dc(int nb, int nc, int nd, bool rows)
 // 160 KB on gfx950).  A block above 80 KB holds its CU's share alone
 // whatever its size, so the whole of it is offered.
 constexpr long long kRowBytes = 160 * 1024;
+// work items of a launch up to which the per-bra kernel's blocks have eight
+// wavefronts and divide an item's components of the first bra shell between
+// them: fewer items than one for every SIMD
+constexpr long long kSplitItems = 1024;
 
 std::atomic<int> g_rows_enabled{1};   // simint_hip_set_jk_rows
 
@@ -407,8 +585,17 @@ hipError_t launch_t(const Launch &L, const JkDev &d, hipStream_t s)
     bool done = false;
     if constexpr (DCR > 0) {
         if (d.K && rbytes <= row_bytes_limit()) {
-            hipLaunchKernelGGL((jk_digest_rows<NB, NC, ND, DCR>), dim3((unsigned)L.nbra), dim3(256), (size_t)rbytes,
-                               s, items, nitems, L.tstart, L.nbra, col, ints, na, d);
+            // a block above half the local data share holds its CU alone: eight
+            // wavefronts, two for every SIMD
+            const long long lbytes = rbytes + 8LL * L.na * NB * 64;
+            const int lanesum = lbytes <= row_bytes_limit();   // room for the lanes' sums of J_ab too
+            const bool few = nitems <= kSplitItems;
+            const int threads = few || lbytes > kRowBytes / 2 ? rows_threads(NB, NC, ND) : 256;
+            const long long share = threads / 64 * (long long)L.nbra / nitems;   // wavefronts an item
+            const int parts = few ? (int)std::max(1LL, std::min<long long>(na, share)) : 1;
+            hipLaunchKernelGGL((jk_digest_rows<NB, NC, ND, DCR>), dim3((unsigned)L.nbra), dim3(threads),
+                               (size_t)(lanesum ? lbytes : rbytes), s, items, nitems, L.tstart, L.nbra, col, ints,
+                               na, parts, lanesum, d);
             done = true;
         }
     }
