@@ -57,6 +57,13 @@ LDS_CU = 160 * 1024
 AREA_GOOD = 22 * 1024    # HRR area up to which four to eight wavefronts share a CU
 SPLIT_GROUPS = 4096      # list launches of at most this many groups share a group
 SPLIT_W = 4              # between so many wavefronts (primitive quartets: up to twice as many)
+# Lists of at most this many groups (four classes side by side then have one
+# a compute unit) share a group's tops between twice as many wavefronts,
+# where that shortens the longest wavefront's work to DEEP_GAIN of it.  The
+# paths to the tops are walked by more of them: about 1.3 times the work in
+# all, so longer lists, which fill the chip, do not.
+DEEP_GROUPS = 64
+DEEP_GAIN = 0.75
 SUM_VALUES = 8           # accumulators added per round where primitive quartets are shared
 # The most AM transferred in the HRR of a class that shares them.  On the
 # mixed-class stream (300000 quartets in a 30-bohr cube) sharing moved
@@ -171,6 +178,7 @@ class Plan:
             if at < self.G:
                 break
             bound += 1
+        self.longest = bound
         self.parts = parts
         self.part_nodes = [set(x for f in p for x in path(f)) for p in self.parts]
         self.nacc = max(len(p) for p in self.parts)
@@ -276,6 +284,22 @@ def split_plan(am):
     return p if 16 * p.lds_doubles <= LDS_CU else plan(am, 1, SPLIT_W)
 
 
+def deep_plan(am):
+    """Plan of the kernel for the shortest lists, or None.  Tops shared in
+    another way leave every value's arithmetic as it is.  Eight wavefronts a
+    workgroup leave 256 registers to each."""
+    ps = split_plan(am)
+    if ps.G == 1:
+        return None
+    try:
+        p = plan(am, 2 * SPLIT_W, 1)
+    except ValueError:
+        return None
+    if p.regs(p.NS) > 240 or p.NQ != ps.NQ or p.longest > DEEP_GAIN * ps.longest:
+        return None
+    return p
+
+
 def base_G(am):
     """Wavefronts a workgroup of the range and long-list kernels: one where
     its HRR area leaves four of them a CU's local data share."""
@@ -306,14 +330,15 @@ def candidate(am):
 
 def emit_cpl(am):
     G = base_G(am)
-    p, ps = plan(am, G), split_plan(am)
+    p, ps, pd = plan(am, G), split_plan(am), deep_plan(am)
     w = _Writer()
     w("// Generated by simint-generator_amd/emitter/hip_cpl.py -- class (%s)" % class_name(am).replace("_", ""))
     w('#include "../device_types.h"')
     w('#include "../boys_device.h"')
     w("")
     w("namespace {")
-    w("constexpr int NE = %d, NPC = %d, QINFO = %d, SPLIT_GROUPS = %d;" % (p.NE, p.npc, QINFO, SPLIT_GROUPS))
+    w("constexpr int NE = %d, NPC = %d, QINFO = %d, SPLIT_GROUPS = %d, DEEP_GROUPS = %d;"
+      % (p.NE, p.npc, QINFO, SPLIT_GROUPS, DEEP_GROUPS))
     w("// per wide component: chain directions, chain exponents, exponents, lane distances to e - 1_d")
     w("__constant__ __attribute__((aligned(16))) unsigned int lane_tab[NE][4] = {")
     for r in p.lane_tables():
@@ -331,18 +356,20 @@ def emit_cpl(am):
     _emit_kernel(p, w, "range")
     _emit_kernel(p, w, "list")
     _emit_kernel(ps, w, "split")
-    _emit_launchers(p, ps, w)
+    if pd:
+        _emit_kernel(pd, w, "deep")
+    _emit_launchers(p, ps, pd, w)
     return w.text()
 
 
 def _emit_kernel(p, w, mode):
     """mode "range": a bra against the kets of a tile; "list": a run of
-    groups of NQ quartets of a list; "split": the same with more wavefronts
-    a group."""
+    groups of NQ quartets of a list; "split", "deep": the same with more
+    wavefronts a group."""
     name = class_name(p.am)
     NS, NQ, G, SW = p.NS, p.NQ, p.G, p.SW
     listmode = mode != "range"
-    kname = {"range": "eri_cpl_%s", "list": "eri_cpll_%s", "split": "eri_cpls_%s"}[mode] % name
+    kname = {"range": "eri_cpl_%s", "list": "eri_cpll_%s", "split": "eri_cpls_%s", "deep": "eri_cpld_%s"}[mode] % name
     w("__global__ void __launch_bounds__(%d, %d) %s(const %s A%s)"
       % (64 * p.W, p.occ, kname, "EriListArgs" if listmode else "EriArgs", ", int groups" if listmode else ""))
     w("{")
@@ -463,7 +490,7 @@ def _emit_kernel(p, w, mode):
     w("")
 
 
-def _emit_launchers(p, ps, w):
+def _emit_launchers(p, ps, pd, w):
     name = class_name(p.am)
     w('extern "C" hipError_t simint_launch_cpl_%s(const EriArgs *a, hipStream_t s)' % name)
     w("{")
@@ -481,6 +508,11 @@ def _emit_launchers(p, ps, w):
     w("    if (a->nquartet <= 0) return hipSuccess;")
     w("    if (a->nquartet > 0x7fff0000LL) return hipErrorInvalidValue;")
     w("    long long ng = (a->nquartet + %d) / %d;" % (ps.NQ - 1, ps.NQ))
+    if pd:
+        w("    if (ng <= DEEP_GROUPS) {")
+        w("        hipLaunchKernelGGL(eri_cpld_%s, dim3((unsigned)ng), dim3(64, %d), 0, s, *a, 1);" % (name, pd.W))
+        w("        return hipGetLastError();")
+        w("    }")
     w("    if (ng <= SPLIT_GROUPS) {")
     w("        hipLaunchKernelGGL(eri_cpls_%s, dim3((unsigned)ng), dim3(64, %d), 0, s, *a, 1);" % (name, ps.W))
     w("        return hipGetLastError();")

@@ -119,3 +119,32 @@ def test_two_stage_recurrence_is_the_graphs(am):
 def test_every_deriv_term_class_is_built():
     assert all(hip_cpl.candidate(am) for am in generate.deriv_term_classes(3))
     assert all(hip_cpl.candidate(am) for am in itertools.product(range(4), repeat=4) if sum(am) >= 9)
+
+
+def test_deep_plans_share_the_tops_in_another_way():
+    """The shortest lists' plans: inside the local data share and 256
+    registers, every top with its path in one wavefront, groups of the same
+    quartets as the short lists' plan, less work for the longest wavefront."""
+    deep = {am: p for am in CLASSES for p in [hip_cpl.deep_plan(am)] if p}
+    assert 40 <= len(deep) and all(sum(am) >= 8 for am in deep)
+    for am, p in deep.items():
+        ps = hip_cpl.split_plan(am)
+        assert ps.G == hip_cpl.SPLIT_W and p.G == 2 * hip_cpl.SPLIT_W and p.SW == 1
+        assert (p.NQ, p.NE) == (ps.NQ, ps.NE) and p.regs(p.NS) <= 240 and p.longest <= 0.75 * ps.longest
+        assert 8 * p.lds_doubles <= hip_cpl.LDS_CU
+        assert p.lds_doubles == p.ent * (p.npc + hip_cpl.QINFO) + p.area
+        assert p.ps > p.NQ * p.NE and p.W * p.npub * p.ps + p.root_doubles(p.ps) <= p.area
+        ks = max(p.nkt, p.ncd) | 1
+        assert p.NQ % p.HQ == 0 and p.cc * p.nch >= p.nab
+        if p.hold:
+            assert p.HQ * p.nkt <= 64 * p.W
+            assert p.HQ * p.nbt * (p.nkt | 1) <= p.area and p.HQ * p.cc * ks <= p.area
+        else:
+            assert p.nch == 1 and p.HQ * max(p.nbt, p.nab) * ks <= p.area
+        assert sorted(f for part in p.parts for f in part) == sorted(p.stops) and len(p.parts) == p.G
+        for part, nodes in zip(p.parts, p.part_nodes):
+            assert len(part) <= p.nacc
+            for f in part:
+                while sum(f):
+                    assert f in nodes
+                    f = step(f, mk_dir(f), -1)
