@@ -142,14 +142,18 @@ class QuartetBatch:
         fork.record(main)
         for s in self._side:
             s.wait_event(fork)
-        # largest classes first, so the long launches start early
-        order = sorted(self.groups, key=lambda g: -g.prim_quartets * (1 + sum(g.cls)) ** 3)
+        # longest classes first, so the long launches start early; a list too
+        # short to fill the chip lasts as long as its deepest quartet.  Every
+        # second round of streams runs backwards: always in the same order,
+        # the first stream would get the longest of every round.
+        order = sorted(self.groups, key=lambda g: -max(g.prim_quartets, 256 * g.kmax) * (1 + sum(g.cls)) ** 3)
         try:
-            for k, g in enumerate(order):
-                L.simint_hip_set_stream(ctypes.c_void_p(self._side[k % n].cuda_stream))
+            for j, g in enumerate(order):
+                k = j % n if j // n % 2 == 0 else n - 1 - j % n
+                L.simint_hip_set_stream(ctypes.c_void_p(self._side[k].cuda_stream))
                 if self.deriv:
                     simint.compute_deriv1_list(g.P, g.Q, g.n, g.idx.data_ptr(), g.idx.data_ptr(),
-                                               g.qout.data_ptr(), self._works[k % n].data_ptr(), d_out,
+                                               g.qout.data_ptr(), self._works[k].data_ptr(), d_out,
                                                self.screen_tol)
                 else:
                     self._list(g, d_out)
