@@ -210,14 +210,14 @@ int   simint_hip_synchronize(void);
 void *simint_hip_stream(void);                /* hipStream_t of the calling thread */
 /* Queue the calling thread's later calls on `stream` (a hipStream_t; NULL:
  * back to the thread's own stream), e.g. to spread the classes of one batch
- * over several streams that a graph capture joins.  The calls that stage
- * host data through the library's per-thread buffers (_prefix, _range,
- * _diag, the drop-in calls) synchronise only the current stream before
- * reusing those buffers: synchronise the previous stream yourself before
- * switching between such calls; list calls take device arrays and need no care. */
+ * over several streams that a graph capture joins.  The range calls
+ * (_prefix, _range, _jk_range, _deriv1_range) queue without waiting and use
+ * the library's per-thread buffers in stream order, also over a change of
+ * stream; _diag and the drop-in calls wait for them first. */
 int   simint_hip_set_stream(void * stream);
 /* Lanes per quartet (1, 2, 4, 8 or 16) of the calling thread's later
- * lane-per-quartet simint_hip_compute_eri_list launches: each lane sums a
+ * lane-per-quartet simint_hip_compute_eri_list launches (and of the terms of
+ * a derivative list): each lane sums a
  * strided share of the quartet's primitive quartets and the shares are added
  * across the lanes before the HRR.  0 (the default): chosen by list length,
  * so that a launch has about 65536 lanes.  Returns the previous setting or

@@ -272,7 +272,10 @@ __global__ void __launch_bounds__(256) jk_digest_t(const WorkItem *items, long l
 // density rows over all a and the integrals of two a at a time (held(): all
 // loads of an a in flight together, each ket's cache lines read while they
 // are in the L1 cache, and a row of the exchange added to the local data
-// share once instead of na times).
+// share once instead of na times).  With this, the loads a step ahead and
+// J_ab summed per lane the digestion of 64 atoms takes 480 ms, 637 before; it
+// is bound by the loads, 64 cache lines an instruction, and the adds into the
+// local data share.
 constexpr int kHeldDoubles = 108;
 constexpr bool held(int nb, int nc, int dc)
 {
@@ -540,7 +543,9 @@ constexpr int pick_dc(int nb, int nc, int nd, bool rows)
 constexpr long long kRowBytes = 160 * 1024;
 // work items of a launch up to which the per-bra kernel's blocks have eight
 // wavefronts and divide an item's components of the first bra shell between
-// them: fewer items than one for every SIMD
+// them: fewer items than one for every SIMD (10 atoms: 4.96 -> 4.80 ms of
+// digestion, which is chains of dependent loads; single components a wavefront
+// took 6.0)
 constexpr long long kSplitItems = 1024;
 
 std::atomic<int> g_rows_enabled{1};   // simint_hip_set_jk_rows

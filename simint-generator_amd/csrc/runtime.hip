@@ -17,7 +17,6 @@
 #include <stdlib.h>
 #include <string.h>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -346,6 +345,16 @@ ThreadCtx &ctx()
     return *c;
 }
 
+// wait until nothing of this thread uses its buffers; fails under capture
+hipError_t idle(ThreadCtx &c)
+{
+    hipError_t e;
+    if ((e = hipStreamSynchronize(c.s)) != hipSuccess) return e;
+    const bool moved = c.range_marked;   // work of an earlier stream
+    if ((e = c.range_enter()) != hipSuccess) return e;
+    return moved ? hipStreamSynchronize(c.s) : hipSuccess;
+}
+
 // ------------------------------------------- host buffers of the drop-in calls
 constexpr size_t kKernelCopy = 1 << 20;   // bytes up to which a kernel does the copy
 constexpr size_t kBackChunk = 4 << 20;    // bytes of one piece on the way back
@@ -380,10 +389,19 @@ hipError_t copy_in(ThreadCtx &c, size_t bytes)
 // slots, each divided among a few threads on its way into the caller's
 // buffer while the next ones cross PCIe: one thread's memcpy (what a copy
 // command to pageable memory does) is several times slower than the link.
+// 180 MB of integrals: 11.5 to 17.6 ms with one copy command, 5.2 so.
 hipError_t copy_back(ThreadCtx &c, double *dst, const double *src, size_t n)
 {
     hipError_t e;
     const size_t bytes = sizeof(double) * n;
+    hipPointerAttribute_t at;
+    if (hipPointerGetAttributes(&at, dst) != hipSuccess) {
+        (void)hipGetLastError();   // pageable memory
+    } else if (at.type == hipMemoryTypeHost || at.type == hipMemoryTypeDevice || at.type == hipMemoryTypeManaged) {
+        // memory the device reaches: one copy, at the link's rate
+        if ((e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, c.s)) != hipSuccess) return e;
+        return hipStreamSynchronize(c.s);
+    }
     if ((e = c.back.reserve(bytes <= kKernelCopy ? bytes : kBackSlots * kBackChunk)) != hipSuccess) return e;
     char *pin = static_cast<char *>(c.back.p);
     if (bytes <= kKernelCopy) {
@@ -426,7 +444,7 @@ hipError_t copy_back(ThreadCtx &c, double *dst, const double *src, size_t n)
     try {
         const int most = std::min<int>(kBackThreads, (int)std::thread::hardware_concurrency() / 2);
         for (; nthread < most; nthread++) helpers[nthread] = std::thread(helper, nthread);
-    } catch (const std::system_error &) {
+    } catch (...) {
         // as many as could be started
     }
     go.store(1, std::memory_order_release);
@@ -980,8 +998,7 @@ int simint_compute_ostei_deriv(int deriv, const simint_multi_shellpair *P, const
     hipError_t e;
     // an earlier asynchronous call of this thread (_range, _prefix, _diag)
     // may still read c.stage or c.split: wait for it before reuse
-    if ((e = hipStreamSynchronize(c.s)) != hipSuccess) { set_err("hipStreamSynchronize", e); return SIMINT_ERROR_HIP; }
-    if ((e = c.range_enter()) != hipSuccess) { set_err("hipStreamWaitEvent", e); return SIMINT_ERROR_HIP; }
+    if ((e = idle(c)) != hipSuccess) { set_err("hipStreamSynchronize", e); return SIMINT_ERROR_HIP; }
     const size_t final_n = (size_t)nP * nQ * nc * (deriv ? 12 : 1);
     const bool gamess = gamess_needed(am);
     const size_t out_bytes = sizeof(double) * (scratch + (deriv ? final_n : 0) + (gamess ? final_n : 0));
@@ -1132,7 +1149,9 @@ namespace {
 constexpr int kMaxTerms = 8;
 constexpr int kExpandLanes = 8;   // threads per bra
 // Work items up to which the terms of a derivative run side by side: eight
-// wavefronts a compute unit.  More fill the chip by themselves.
+// wavefronts a compute unit.  More fill the chip by themselves.  8, 12 and 16
+// atoms: 33.7, 47.5 and 75.6 ms one behind another, 29.2, 40.8 and 68.2 so;
+// without a limit 40.6 and 68.1, so nothing is to be had above it.
 constexpr long long kForkItems = 2048;
 
 // What a range launch covers, in pinned host memory: per bra its ket range,
@@ -1402,8 +1421,7 @@ long long simint_hip_compute_eri_diag(const simint_hip_pairs *P, double *d_out)
         items[b].obase = 0;
     }
     hipError_t e;
-    if ((e = hipStreamSynchronize(c.s)) != hipSuccess) { set_err("hipStreamSynchronize", e); return SIMINT_ERROR_HIP; }
-    if ((e = c.range_enter()) != hipSuccess) { set_err("hipStreamWaitEvent", e); return SIMINT_ERROR_HIP; }
+    if ((e = idle(c)) != hipSuccess) { set_err("hipStreamSynchronize", e); return SIMINT_ERROR_HIP; }
     const size_t bytes = sizeof(WorkItem) * items.size();
     if ((e = c.stage.reserve(bytes)) != hipSuccess) { set_err("hipHostMalloc", e); return SIMINT_ERROR_HIP; }
     if ((e = c.items.reserve(bytes)) != hipSuccess) { set_err("hipMalloc", e); return SIMINT_ERROR_HIP; }
@@ -1580,7 +1598,10 @@ long long deriv1_list(const simint_hip_pairs *P, const simint_hip_pairs *Q, long
         }
         a.out = d_work + t.off * nquartet;
         a.ostride = t.nc;
-        a.split = list_split(nquartet);
+        // several lanes a quartet add its primitive quartets in another order,
+        // which the HRR and the weight 2a amplify: only where the HRR transfers
+        // one unit of AM at most (six (sd|pp) quartets on a lane each took 1.2 ms)
+        if (std::min(t.am[0], t.am[1]) + std::min(t.am[2], t.am[3]) <= 1) a.split = list_split(nquartet);
         if ((e = fns[k](&a, c.s)) != hipSuccess) { set_err("class kernel launch", e); return SIMINT_ERROR_HIP; }
         if (t.sign > 0) d.plus[t.centre] = a.out;
         else d.minus[t.centre] = a.out;

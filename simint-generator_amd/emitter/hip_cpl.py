@@ -61,15 +61,18 @@ SPLIT_W = 4              # between so many wavefronts (primitive quartets: up to
 # a compute unit) share a group's tops between twice as many wavefronts,
 # where that shortens the longest wavefront's work to DEEP_GAIN of it.  The
 # paths to the tops are walked by more of them: about 1.3 times the work in
-# all, so longer lists, which fill the chip, do not.
+# all, so longer lists, which fill the chip, do not.  256 classes of 32
+# quartets: 13.4 ms with four wavefronts a group, 12.6 with eight.
 DEEP_GROUPS = 64
 DEEP_GAIN = 0.75
 SUM_VALUES = 8           # accumulators added per round where primitive quartets are shared
 # The most AM transferred in the HRR of a class that shares them.  On the
 # mixed-class stream (300000 quartets in a 30-bohr cube) sharing moved
-# integrals of classes above it by up to 8e-6 of the set's root mean square
-# (8e-9 of its norm), of the others by at most 1e-10.
-SHARE_AM = 3
+# integrals of classes above 3 by up to 8e-6 of the set's root mean square
+# (8e-9 of its norm), of the others by at most 1e-10; but as terms of first
+# derivatives, weighted by 2a, classes of 3 moved 1500 derivatives by up to
+# 2e-8 of their norm, classes of 2 by 3e-11 (12 seeds).
+SHARE_AM = 1
 
 # primitive-quartet block of the local data share, in doubles
 P_E, P_ID, P_EOVER, P_EO2, P_S, P_SOVER, P_SO2, P_O2PQ, P_F = 0, 6, 8, 9, 10, 16, 17, 18, 20

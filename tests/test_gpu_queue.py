@@ -124,5 +124,12 @@ def test_results_to_the_host(gpu, nbra, nket):
     assert rc == nbra * nket
     assert np.isnan(got[-1])
     assert np.array_equal(got[:-1], dev.cpu().numpy())
+    # and into memory the device reaches itself
+    for kw in ({"pin_memory": True}, {"device": "cuda"}):
+        into = torch.full((nv,), float("nan"), dtype=torch.float64, **kw)
+        torch.cuda.synchronize()
+        assert simint.lib().simint_compute_eri(ctypes.byref(hp.mp), ctypes.byref(hq.mp), 0.0, None,
+                                               ctypes.cast(into.data_ptr(), simint.dptr)) == nbra * nket
+        assert torch.equal(into.cpu(), dev.cpu())
     for h in (P, Q, hp, hq, bb, bk):
         h.free()
