@@ -71,8 +71,10 @@ SUM_VALUES = 8           # accumulators added per round where primitive quartets
 # integrals of classes above 3 by up to 8e-6 of the set's root mean square
 # (8e-9 of its norm), of the others by at most 1e-10; but as terms of first
 # derivatives, weighted by 2a, classes of 3 moved 1500 derivatives by up to
-# 2e-8 of their norm, classes of 2 by 3e-11 (12 seeds).
-SHARE_AM = 1
+# 2e-8 of their norm, classes of 2 by 3e-11, of 1 by 4e-13 (12 seeds).  What
+# it is worth, with limits of 3, 2 and 1: 8192 quartets 12.8, 16.0 and 20.4
+# ms, 300000 quartets 44.2, 47.8 and 52.9, 1500 derivatives 48, 66 and 83.
+SHARE_AM = 2
 
 # primitive-quartet block of the local data share, in doubles
 P_E, P_ID, P_EOVER, P_EO2, P_S, P_SOVER, P_SO2, P_O2PQ, P_F = 0, 6, 8, 9, 10, 16, 17, 18, 20

@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("am,deriv", [((2, 2, 2, 2), 0), ((3, 2, 3, 3), 0), ((3, 3, 3, 1), 0), ((2, 2, 3, 3), 0),
-                                      ((3, 3, 3, 3), 0), ((3, 1, 2, 2), 0), ((2, 1, 2, 1), 0),
+                                      ((3, 3, 3, 3), 0), ((3, 1, 2, 2), 0), ((2, 2, 2, 1), 0),
                                       ((3, 3, 2, 1), 1)])
 def test_shortest_lists_equal_longer_ones(gpu, am, deriv):
     shells = _pool(seed=4, per_am=6, maxk=3)
