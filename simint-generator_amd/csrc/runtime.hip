@@ -1816,7 +1816,8 @@ hipError_t thread_buffers(size_t host_bytes, size_t in_bytes, size_t out_bytes, 
 {
     ThreadCtx &c = ctx();
     hipError_t e;
-    if ((e = hipStreamSynchronize(c.s)) != hipSuccess) return e;
+    // a diag call queued on this stream or on one left since may still read c.stage
+    if ((e = idle(c)) != hipSuccess) return e;
     if ((e = c.stage.reserve(host_bytes)) != hipSuccess) return e;
     if ((e = c.in.reserve(in_bytes)) != hipSuccess) return e;
     if ((e = c.out.reserve(out_bytes)) != hipSuccess) return e;
