@@ -213,7 +213,10 @@ void *simint_hip_stream(void);                /* hipStream_t of the calling thre
  * over several streams that a graph capture joins.  The range calls
  * (_prefix, _range, _jk_range, _deriv1_range) queue without waiting and use
  * the library's per-thread buffers in stream order, also over a change of
- * stream; _diag and the drop-in calls wait for them first. */
+ * stream; _diag and the drop-in calls wait for them first.  The stream that
+ * is left is not touched any more and may already be destroyed.  (If it is the
+ * thread's own stream and the caller began a capture on it other than by
+ * simint_hip_capture_begin, the next of these calls waits for the device.) */
 int   simint_hip_set_stream(void * stream);
 /* Lanes per quartet (1, 2, 4, 8 or 16) of the calling thread's later
  * lane-per-quartet simint_hip_compute_eri_list launches (and of the terms of

@@ -267,9 +267,10 @@ struct ThreadCtx {
     // stream their device buffers (items, split) are reused in order.
     PinRing ring;
     hipEvent_t range_ev = nullptr;
-    bool range_live = false;     // range work queued on s since s was taken up
-    bool range_marked = false;   // range_ev stands behind such work of an earlier stream
-    bool range_lost = false;     // such work was left on a stream that was being captured
+    bool range_live = false;     // range work queued on own with no event behind it yet
+    bool range_marked = false;   // range_ev stands behind the last range work
+    bool range_here = false;     // ... which is on s, queued since s was taken up
+    bool range_lost = false;     // own was left with range work on it while it was being captured
     ThreadCtx()
     {
         hipStreamCreateWithFlags(&own, hipStreamNonBlocking);
@@ -294,26 +295,40 @@ struct ThreadCtx {
         }
         return hipEventCreateWithFlags(&fork_ev, hipEventDisableTiming);
     }
-    // before s is left, or its work is captured: the range work queued on it
-    // ends at range_ev
-    hipError_t range_leave()
+    // After range work has been queued on s.  A caller's stream gets the event
+    // at once: the caller may destroy it before the next call here, so it is
+    // not touched later.  own always lives: its event waits until it is left.
+    void range_done()
     {
-        if (!range_live) return hipSuccess;
-        hipError_t e;
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if ((e = hipStreamIsCapturing(s, &cap)) != hipSuccess) return e;
-        if (cap != hipStreamCaptureStatusNone) {   // no event can be recorded but into the graph
-            range_live = false;
-            range_lost = true;
-            return hipSuccess;
+        if (s == own) {
+            range_live = true;
+            return;
         }
-        if (!range_ev && (e = hipEventCreateWithFlags(&range_ev, hipEventDisableTiming)) != hipSuccess) return e;
-        if ((e = hipEventRecord(range_ev, s)) != hipSuccess) return e;
-        range_live = false;
-        range_marked = true;
-        return hipSuccess;
+        hipError_t e = hipSuccess;
+        if (!range_ev) e = hipEventCreateWithFlags(&range_ev, hipEventDisableTiming);
+        if (e == hipSuccess) e = hipEventRecord(range_ev, s);
+        if (e != hipSuccess) {   // no event: nothing may be left
+            hipStreamSynchronize(s);
+            return;
+        }
+        range_marked = range_here = true;
     }
-    // before items or split are used on s
+    // before s is left, or its work is captured
+    void range_leave()
+    {
+        range_here = false;
+        if (!range_live) return;
+        range_live = false;
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        hipError_t e = hipStreamIsCapturing(own, &cap);
+        // under a capture that the caller began, no event can be recorded but into the graph
+        if (e == hipSuccess && cap != hipStreamCaptureStatusNone) e = hipErrorStreamCaptureUnsupported;
+        if (e == hipSuccess && !range_ev) e = hipEventCreateWithFlags(&range_ev, hipEventDisableTiming);
+        if (e == hipSuccess) e = hipEventRecord(range_ev, own);
+        if (e == hipSuccess) range_marked = true;
+        else range_lost = true;
+    }
+    // before the range buffers are used on s
     hipError_t range_enter()
     {
         if (range_lost) {
@@ -321,12 +336,11 @@ struct ThreadCtx {
             if (e != hipSuccess) return e;
             range_lost = false;
         }
-        if (range_marked) {
+        if (range_marked && !range_here) {
             const hipError_t e = hipStreamWaitEvent(s, range_ev, 0);
             if (e != hipSuccess) return e;
             range_marked = false;
         }
-        range_live = true;
         return hipSuccess;
     }
     // device memory that work queued on s may still use, grown when it must be
@@ -345,12 +359,18 @@ ThreadCtx &ctx()
     return *c;
 }
 
+// range_done() on every way out, once range work may have been queued
+struct RangeDone {
+    ThreadCtx &c;
+    ~RangeDone() { c.range_done(); }
+};
+
 // wait until nothing of this thread uses its buffers; fails under capture
 hipError_t idle(ThreadCtx &c)
 {
     hipError_t e;
     if ((e = hipStreamSynchronize(c.s)) != hipSuccess) return e;
-    const bool moved = c.range_marked;   // work of an earlier stream
+    const bool moved = c.range_marked && !c.range_here;   // work of an earlier stream
     if ((e = c.range_enter()) != hipSuccess) return e;
     return moved ? hipStreamSynchronize(c.s) : hipSuccess;
 }
@@ -1012,6 +1032,7 @@ int simint_compute_ostei_deriv(int deriv, const simint_multi_shellpair *P, const
     for (auto &t : terms) nst = std::max(nst, (size_t)simint_dispatch_staging(t.am[0], t.am[1], t.am[2], t.am[3]));
     if (nst && (e = c.split.reserve(sizeof(double) * nst * SIMINT_TILE * (size_t)nit)) != hipSuccess) {
         set_err("hipMalloc", e);
+        hipStreamSynchronize(c.s);   // the copy out of c.stage
         return SIMINT_ERROR_HIP;
     }
     char *base = static_cast<char *>(c.in.p);
@@ -1241,6 +1262,7 @@ long long range_launch(const simint_hip_pairs *P, const simint_hip_pairs *Q, int
         return SIMINT_ERROR_HIP;
     }
     if ((e = c.range_enter()) != hipSuccess) { set_err("hipStreamWaitEvent", e); return SIMINT_ERROR_HIP; }
+    const RangeDone done{c};
     size_t nst = 0;
     for (int t = 0; t < nterm; t++)
         nst = std::max(nst, (size_t)simint_dispatch_staging(terms[t].am[0], terms[t].am[1], terms[t].am[2],
@@ -1390,6 +1412,7 @@ long long simint_hip_compute_jk_range(const simint_hip_pairs *P, const simint_hi
     if (nq <= 0 || nitems == 0 || (!jk->J && !jk->K)) return nq;
     const hipError_t e = simint_rt::launch_jk_digest(t.am, items, nitems, tstart, nbra, Q->til.col, d_out, jk,
                                                      ctx().s);
+    ctx().range_done();   // the digestion reads the items too
     if (e != hipSuccess) { set_err("digest launch", e); return SIMINT_ERROR_HIP; }
     return nq;
 }
@@ -1422,6 +1445,7 @@ long long simint_hip_compute_eri_diag(const simint_hip_pairs *P, double *d_out)
     }
     hipError_t e;
     if ((e = idle(c)) != hipSuccess) { set_err("hipStreamSynchronize", e); return SIMINT_ERROR_HIP; }
+    const RangeDone done{c};
     const size_t bytes = sizeof(WorkItem) * items.size();
     if ((e = c.stage.reserve(bytes)) != hipSuccess) { set_err("hipHostMalloc", e); return SIMINT_ERROR_HIP; }
     if ((e = c.items.reserve(bytes)) != hipSuccess) { set_err("hipMalloc", e); return SIMINT_ERROR_HIP; }
@@ -1724,9 +1748,8 @@ struct simint_hip_graph {
 int simint_hip_capture_begin(void)
 {
     if (!ensure_device()) return SIMINT_ERROR_NO_DEVICE;
-    hipError_t e = ctx().range_leave();
-    if (e != hipSuccess) { set_err("hipEventRecord", e); return SIMINT_ERROR_HIP; }
-    e = hipStreamBeginCapture(ctx().s, hipStreamCaptureModeThreadLocal);
+    ctx().range_leave();
+    hipError_t e = hipStreamBeginCapture(ctx().s, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) { set_err("hipStreamBeginCapture", e); return SIMINT_ERROR_HIP; }
     return 0;
 }
@@ -1791,12 +1814,8 @@ int simint_hip_set_stream(void *stream)
 {
     if (!ensure_device()) return SIMINT_ERROR_NO_DEVICE;
     ThreadCtx &c = ctx();
-    const hipStream_t to = stream ? static_cast<hipStream_t>(stream) : c.own;
-    if (to != c.s) {
-        const hipError_t e = c.range_leave();
-        if (e != hipSuccess) { set_err("hipEventRecord", e); return SIMINT_ERROR_HIP; }
-    }
-    c.s = to;
+    c.range_leave();
+    c.s = stream ? static_cast<hipStream_t>(stream) : c.own;
     return 0;
 }
 
