@@ -10,6 +10,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <condition_variable>
 #include <memory>
 #include <mutex>
 #include <numeric>
@@ -260,9 +261,7 @@ struct ThreadCtx {
     DevBuf in, out, items;
     DevBuf split;      // staging of the split lane-per-quartet kernels
     PinBuf stage;
-    PinBuf back;                    // results on their way to a caller's buffer
-    static constexpr int kSlots = 4;
-    hipEvent_t back_ev[kSlots] = {};     // per slot of it: the copy into it is done
+    PinBuf back;       // small results on their way to a caller's buffer
     // Range launches queue without waiting for the ones before: on one
     // stream their device buffers (items, split) are reused in order.
     PinRing ring;
@@ -378,8 +377,24 @@ hipError_t idle(ThreadCtx &c)
 // ------------------------------------------- host buffers of the drop-in calls
 constexpr size_t kKernelCopy = 1 << 20;   // bytes up to which a kernel does the copy
 constexpr size_t kBackChunk = 4 << 20;    // bytes of one piece on the way back
-constexpr int kBackSlots = ThreadCtx::kSlots;
+constexpr int kBackSlots = 4;
 constexpr int kBackThreads = 5;           // beside the calling thread
+
+// The pinned slots large results cross PCIe through, and per slot the event
+// behind the copy into it.  One for the process: a call that finds them in
+// use takes the plain copy command, so however many threads call, the slots
+// are 16 MiB and the copying threads five.
+struct BackRing {
+    std::mutex m;
+    PinBuf b;
+    hipEvent_t ev[kBackSlots] = {};
+};
+
+BackRing &back_ring()
+{
+    static BackRing *r = new BackRing;   // not released, as ThreadCtx
+    return *r;
+}
 
 __global__ void __launch_bounds__(256) copy_words(const double *__restrict__ from, double *__restrict__ to, size_t n)
 {
@@ -409,7 +424,8 @@ hipError_t copy_in(ThreadCtx &c, size_t bytes)
 // slots, each divided among a few threads on its way into the caller's
 // buffer while the next ones cross PCIe: one thread's memcpy (what a copy
 // command to pageable memory does) is several times slower than the link.
-// 180 MB of integrals: 11.5 to 17.6 ms with one copy command, 5.2 so.
+// 180 MB of integrals: 11.5 to 17.6 ms with one copy command, 5.2 so.  The
+// threads sleep until the first piece has arrived.
 hipError_t copy_back(ThreadCtx &c, double *dst, const double *src, size_t n)
 {
     hipError_t e;
@@ -422,15 +438,23 @@ hipError_t copy_back(ThreadCtx &c, double *dst, const double *src, size_t n)
         if ((e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, c.s)) != hipSuccess) return e;
         return hipStreamSynchronize(c.s);
     }
-    if ((e = c.back.reserve(bytes <= kKernelCopy ? bytes : kBackSlots * kBackChunk)) != hipSuccess) return e;
-    char *pin = static_cast<char *>(c.back.p);
     if (bytes <= kKernelCopy) {
+        if ((e = c.back.reserve(bytes)) != hipSuccess) return e;
+        char *pin = static_cast<char *>(c.back.p);
         if ((e = launch_copy_words(src, pin, n, c.s)) != hipSuccess) return e;
         if ((e = hipStreamSynchronize(c.s)) != hipSuccess) return e;
         memcpy(dst, pin, bytes);
         return hipSuccess;
     }
-    for (hipEvent_t &ev : c.back_ev)
+    BackRing &ring = back_ring();
+    const std::unique_lock<std::mutex> mine(ring.m, std::try_to_lock);
+    if (!mine) {
+        if ((e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c.s)) != hipSuccess) return e;
+        return hipStreamSynchronize(c.s);
+    }
+    if ((e = ring.b.reserve(kBackSlots * kBackChunk)) != hipSuccess) return e;
+    char *pin = static_cast<char *>(ring.b.p);
+    for (hipEvent_t &ev : ring.ev)
         if (!ev && (e = hipEventCreateWithFlags(&ev, hipEventDisableTiming)) != hipSuccess) return e;
     const long long npiece = (long long)((bytes + kBackChunk - 1) / kBackChunk);
     auto piece_bytes = [&](long long k) { return std::min(kBackChunk, bytes - (size_t)k * kBackChunk); };
@@ -438,7 +462,7 @@ hipError_t copy_back(ThreadCtx &c, double *dst, const double *src, size_t n)
         const hipError_t r = hipMemcpyAsync(pin + (size_t)(k % kBackSlots) * kBackChunk,
                                             reinterpret_cast<const char *>(src) + (size_t)k * kBackChunk,
                                             piece_bytes(k), hipMemcpyDeviceToHost, c.s);
-        return r != hipSuccess ? r : hipEventRecord(c.back_ev[k % kBackSlots], c.s);
+        return r != hipSuccess ? r : hipEventRecord(ring.ev[k % kBackSlots], c.s);
     };
     std::atomic<long long> ready{0};                       // pieces that have arrived (-1: give up)
     std::atomic<long long> copied[kBackThreads] = {};      // pieces each thread is done with
@@ -449,9 +473,14 @@ hipError_t copy_back(ThreadCtx &c, double *dst, const double *src, size_t n)
         memcpy(reinterpret_cast<char *>(dst) + (size_t)k * kBackChunk + lo,
                pin + (size_t)(k % kBackSlots) * kBackChunk + lo, hi - lo);
     };
-    std::atomic<int> go{0};
+    std::mutex start_m;
+    std::condition_variable start;
+    bool go = false;
     auto helper = [&](int t) {
-        while (!go.load(std::memory_order_acquire)) std::this_thread::yield();
+        {
+            std::unique_lock<std::mutex> lk(start_m);
+            start.wait(lk, [&] { return go; });
+        }
         for (long long k = 0; k < npiece; k++) {
             long long r;
             while ((r = ready.load(std::memory_order_acquire)) >= 0 && r <= k) std::this_thread::yield();
@@ -467,12 +496,19 @@ hipError_t copy_back(ThreadCtx &c, double *dst, const double *src, size_t n)
     } catch (...) {
         // as many as could be started
     }
-    go.store(1, std::memory_order_release);
+    auto wake = [&] {
+        {
+            const std::lock_guard<std::mutex> lk(start_m);
+            go = true;
+        }
+        start.notify_all();
+    };
     e = hipSuccess;
     for (long long k = 0; k < std::min<long long>(kBackSlots, npiece) && e == hipSuccess; k++) e = queue(k);
     for (long long k = 0; k < npiece && e == hipSuccess; k++) {
-        if ((e = hipEventSynchronize(c.back_ev[k % kBackSlots])) != hipSuccess) break;
+        if ((e = hipEventSynchronize(ring.ev[k % kBackSlots])) != hipSuccess) break;
         ready.store(k + 1, std::memory_order_release);
+        if (k == 0) wake();
         part(k, nthread);
         if (k + kBackSlots < npiece) {
             for (int t = 0; t < nthread; t++)
@@ -480,7 +516,11 @@ hipError_t copy_back(ThreadCtx &c, double *dst, const double *src, size_t n)
             e = queue(k + kBackSlots);
         }
     }
-    if (e != hipSuccess) ready.store(-1, std::memory_order_release);
+    if (e != hipSuccess) {
+        ready.store(-1, std::memory_order_release);
+        wake();
+        hipStreamSynchronize(c.s);   // nothing may still write to the slots when another call takes them
+    }
     for (int t = 0; t < nthread; t++) helpers[t].join();
     return e;
 }
