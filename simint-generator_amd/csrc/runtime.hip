@@ -274,25 +274,33 @@ struct ThreadCtx {
     {
         hipStreamCreateWithFlags(&own, hipStreamNonBlocking);
         s = own;
-        // now, not when first needed: streams are dealt out over the few
-        // hardware queues in the order of their creation, and these are to
-        // have other queues than own
-        make_side();
+        side_streams();
     }
-    // side streams for the terms of one derivative range
     static constexpr int kSide = 3;
-    hipStream_t side[kSide] = {};
     hipEvent_t fork_ev = nullptr, join_ev[kSide] = {};
-    hipError_t make_side()
+    // The side streams for the terms of a derivative range, null if they could
+    // not be made.  The process has them once: streams are dealt out over the
+    // few hardware queues in the order of their creation, so with three of its
+    // own for every thread all threads' own streams came to share one queue
+    // (two threads' calls of 256 x 256 (pp) pairs of depth 8: 16.8 ms side by
+    // side, 20.8 so).  Made with the first thread's own stream, which is to
+    // have another queue than they.
+    static const hipStream_t *side_streams()
     {
-        if (fork_ev) return hipSuccess;
+        static hipStream_t side[kSide];
+        static const bool made = [] {
+            for (hipStream_t &s : side)
+                if (hipStreamCreateWithFlags(&s, hipStreamNonBlocking) != hipSuccess) return false;
+            return true;
+        }();
+        return made ? side : nullptr;
+    }
+    hipError_t make_events()
+    {
         hipError_t e;
-        for (int k = 0; k < kSide; k++) {
-            if (!side[k] && (e = hipStreamCreateWithFlags(&side[k], hipStreamNonBlocking)) != hipSuccess) return e;
-            if (!join_ev[k] && (e = hipEventCreateWithFlags(&join_ev[k], hipEventDisableTiming)) != hipSuccess)
-                return e;
-        }
-        return hipEventCreateWithFlags(&fork_ev, hipEventDisableTiming);
+        for (hipEvent_t *ev : {&fork_ev, &join_ev[0], &join_ev[1], &join_ev[2]})
+            if (!*ev && (e = hipEventCreateWithFlags(ev, hipEventDisableTiming)) != hipSuccess) return e;
+        return hipSuccess;
     }
     // After range work has been queued on s.  A caller's stream gets the event
     // at once: the caller may destroy it before the next call here, so it is
@@ -1354,9 +1362,10 @@ long long range_launch(const simint_hip_pairs *P, const simint_hip_pairs *Q, int
     hipLaunchKernelGGL(expand_range_items, dim3(nblk, nterm), dim3(256), 0, c.s, x);
     if ((e = hipGetLastError()) != hipSuccess) { set_err("expand launch", e); return SIMINT_ERROR_HIP; }
     // stream of each term: 0 is c.s, k > 0 side stream k - 1
+    const hipStream_t *const side = ThreadCtx::side_streams();
     int on[kMaxTerms] = {};
     bool used[ThreadCtx::kSide + 1] = {};
-    if (nterm > 1 && nitems <= kForkItems) {
+    if (nterm > 1 && nitems <= kForkItems && side) {
         double load[ThreadCtx::kSide + 1] = {};
         int order[kMaxTerms];
         double cost[kMaxTerms];
@@ -1374,9 +1383,9 @@ long long range_launch(const simint_hip_pairs *P, const simint_hip_pairs *Q, int
             load[on[order[k]]] += cost[order[k]];
             used[on[order[k]]] = true;
         }
-        if ((e = c.make_side()) == hipSuccess) e = hipEventRecord(c.fork_ev, c.s);
+        if ((e = c.make_events()) == hipSuccess) e = hipEventRecord(c.fork_ev, c.s);
         for (int k = 0; k < ThreadCtx::kSide && e == hipSuccess; k++)
-            if (used[k + 1]) e = hipStreamWaitEvent(c.side[k], c.fork_ev, 0);
+            if (used[k + 1]) e = hipStreamWaitEvent(side[k], c.fork_ev, 0);
         if (e != hipSuccess) { set_err("side streams", e); return SIMINT_ERROR_HIP; }
     }
     hipError_t failed = hipSuccess;
@@ -1397,13 +1406,13 @@ long long range_launch(const simint_hip_pairs *P, const simint_hip_pairs *Q, int
         a.tol2 = (screen_tol > 0.0 && P->has_screen && Q->has_screen) ? screen_tol * screen_tol : 0.0;
         a.ket_screen_max = Q->screen_max;
         a.stride = x.stride[t];
-        failed = T.fn(&a, on[t] ? c.side[on[t] - 1] : c.s);
+        failed = T.fn(&a, on[t] ? side[on[t] - 1] : c.s);
     }
     for (int k = 0; k < ThreadCtx::kSide; k++) {
         if (!used[k + 1]) continue;
-        if ((e = hipEventRecord(c.join_ev[k], c.side[k])) == hipSuccess) e = hipStreamWaitEvent(c.s, c.join_ev[k], 0);
+        if ((e = hipEventRecord(c.join_ev[k], side[k])) == hipSuccess) e = hipStreamWaitEvent(c.s, c.join_ev[k], 0);
         if (e != hipSuccess) {   // nothing of the call may run on beside what is queued after it
-            hipStreamSynchronize(c.side[k]);
+            hipStreamSynchronize(side[k]);
             if (failed == hipSuccess) failed = e;
         }
     }
