@@ -235,7 +235,14 @@ const char *simint_hip_last_error(void);
  * device staging area), 5 / 6 = the same over ket tops, 7 = component-lane
  * (one lane per component of the wider side), 0 = class not built.  The setter lets a caller (the
  * autotuner, tests) pick a family; it returns the previous one or a
- * negative value if that family is not built for the class. */
+ * negative value if that family is not built for the class.  Launches of few
+ * items (a bra pair against up to 64 kets) run other kernels of family 1:
+ * where the class has no HRR, or only one that the other side's shells s leave
+ * alone, several wavefronts share an item's primitive quartets; the other
+ * classes run the component-lane kernel where it is built, in FP64 also for
+ * precision 1.  The values are family 1's bit for bit, except that without
+ * HRR the primitive quartets are summed in up to eight parts: there they can
+ * differ in the last places between launches of few and of many items. */
 int simint_hip_class_kernel(int la, int lb, int lc, int ld);
 int simint_hip_set_class_kernel(int la, int lb, int lc, int ld, int family);
 /* The same for the quartet-list calls: 1 = lane-per-quartet, 2 = wave-per-quartet,
