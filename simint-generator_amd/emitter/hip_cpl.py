@@ -465,6 +465,11 @@ def _emit_kernel(p, w, mode):
     w("            " + (sync if SW == 1 else fence))
     _emit_setup(p, w, listmode)
     w("            " + (sync if SW == 1 else fence))
+    if G > 1:
+        w("            if (screen) alive = (unsigned)__builtin_amdgcn_readfirstlane((int)((const unsigned *)qi)[14]);")
+    w("            unsigned every = 0;   // primitive quartet 0 of every quartet of a group")
+    w("#pragma unroll")
+    w("            for (int v = 0; v < NQ; ++v) every |= 1u << (v * PBK);")
     if SW > 1:
         w("            const int gi = 0;")
     else:
@@ -475,6 +480,7 @@ def _emit_kernel(p, w, mode):
             w("                if (wave == %d) {" % part)
         w("#pragma unroll 1")
         w("                for (int pp = 0; pp < npb_; ++pp) {")
+        w("                    if (((alive >> (gi * NQ * PBK + pp)) & every) == 0) continue;")
         _emit_vrr(p, w, part)
         w("                }")
         if G > 1:
@@ -537,20 +543,36 @@ def _emit_setup(p, w, listmode):
     bra_pa = "pa" if g.bra_j else "pb"
     ket_pa = "pa" if g.ket_l else "pb"
     ind = "                "
-    w("            if (%s < GB * NQ * PBK) {" % ("lane" if p.SW > 1 else "tid"))
-    w(ind + "const int r = lane / PBK, pl = p0 + lane - r * PBK;")
-    w(ind + "const int qx = q_first + g0 * NQ + r;")
-    w(ind + "const int q = qx < q_end ? qx : q_end - 1;")
+    w("            const bool mine = %s < GB * NQ * PBK;" % ("lane" if p.SW > 1 else "tid"))
+    w("            bool live = false;")
+    w("            const int r = lane / PBK, pl = p0 + lane - r * PBK;")
+    w("            const int qx = q_first + g0 * NQ + r;")
+    w("            const int q = qx < q_end ? qx : q_end - 1;")
     if not listmode:
-        w(ind + "const bool live = qx < q_end && pl < npb * nq;")
-        w(ind + "const int i = live ? ib0 + pl / nq : 0;")
-        w(ind + "const long long kj = live ? kt + q + (long long)SIMINT_TILE * (pl % nq) : 0;")
+        w("            int i = 0;")
+        w("            long long kj = 0;")
+        w("            if (mine) {")
+        w(ind + "live = qx < q_end && pl < npb * nq;")
+        w(ind + "if (live) {")
+        w(ind + "    i = ib0 + pl / nq;")
+        w(ind + "    kj = kt + q + (long long)SIMINT_TILE * (pl % nq);")
     else:
-        w(ind + "const int bp = A.qbra[q], kp = A.qket[q];")
+        w("            int i = 0, kj = 0, bp = 0, kp = 0;")
+        w("            if (mine) {")
+        w(ind + "bp = A.qbra[q], kp = A.qket[q];")
         w(ind + "const int nq = A.ket.np[kp];")
-        w(ind + "const bool live = qx < q_end && pl < A.bra.np[bp] * nq;")
-        w(ind + "const int i = live ? A.bra.poff[bp] + pl / nq : 0;")
-        w(ind + "const int kj = live ? A.ket.poff[kp] + pl % nq : 0;")
+        w(ind + "live = qx < q_end && pl < A.bra.np[bp] * nq;")
+        w(ind + "if (live) {")
+        w(ind + "    i = A.bra.poff[bp] + pl / nq;")
+        w(ind + "    kj = A.ket.poff[kp] + pl % nq;")
+    w(ind + "    if (screen && (A.bra.screen[i] * A.ket_screen_max < A.tol2 ||")
+    w(ind + "                   A.bra.screen[i] * A.ket.screen[kj] < A.tol2)) live = false;")
+    w(ind + "}")
+    w("            }")
+    # 16 lanes at most: a primitive quartet that is screened in every quartet
+    # of the group is left out, and the preparation of a batch of such
+    w("            %s = screen ? (unsigned)__ballot(live) : ~0u;" % ("unsigned alive" if p.G > 1 else "const unsigned alive"))
+    w("            if (alive != 0 && mine) {")
     w(ind + "double P_alpha = 1.0, P_inv = 1.0, P_prefac = 0.0, Q_alpha = 1.0, Q_inv = 1.0, Q_prefac = 0.0;")
     w(ind + "double PA0 = 0.0, PA1 = 0.0, PA2 = 0.0, QC0 = 0.0, QC1 = 0.0, QC2 = 0.0, PQx = 0.0, PQy = 0.0, PQz = 0.0;")
     w(ind + "if (live) {")
@@ -561,8 +583,6 @@ def _emit_setup(p, w, listmode):
     w(ind + "    PQx = A.bra.x[i] - A.ket.x[kj];")
     w(ind + "    PQy = A.bra.y[i] - A.ket.y[kj];")
     w(ind + "    PQz = A.bra.z[i] - A.ket.z[kj];")
-    w(ind + "    if (screen && (A.bra.screen[i] * A.ket_screen_max < A.tol2 ||")
-    w(ind + "                   A.bra.screen[i] * A.ket.screen[kj] < A.tol2)) P_prefac = 0.0;")
     w(ind + "}")
     w(ind + "const double PQalpha_mul = P_alpha * Q_alpha;")
     w(ind + "const double PQalpha_sum = P_alpha + Q_alpha;")
@@ -592,19 +612,21 @@ def _emit_setup(p, w, listmode):
     put(P_O2PQ, "0.5 * one_over_PQalpha_sum", "0.0")
     for m in range(0, p.L + 1, 2):
         put(P_F + m, "F[%d] * prefac" % m, "F[%d] * prefac" % (m + 1) if m < p.L else "0.0")
-    # the quartet's block: with its first primitive of every batch
-    w(ind + "if (lane == r * PBK) {")
-    w(ind + "    double *const h = %s + r * QINFO;" % ("qmine" if p.SW > 1 else "qi"))
+    w("            }")
+    # the quartet's block for the HRR: with the last batch
+    w("            if (mine && lane == r * PBK && p0 + PBK >= p_end) {")
+    w(ind + "double *const h = %s + r * QINFO;" % ("qmine" if p.SW > 1 else "qi"))
     b, k = ("wi.bra", "(long long)wi.tile * SIMINT_TILE + q") if not listmode else ("bp", "kp")
     for c in range(3):
-        w(ind + "    h[%d] = A.bra.ab%s[%s];" % (c, "xyz"[c], b))
-        w(ind + "    h[%d] = A.ket.ab%s[%s];" % (3 + c, "xyz"[c], k))
+        w(ind + "h[%d] = A.bra.ab%s[%s];" % (c, "xyz"[c], b))
+        w(ind + "h[%d] = A.ket.ab%s[%s];" % (3 + c, "xyz"[c], k))
     if listmode:
-        w(ind + "    ((long long *)h)[6] = A.qout ? A.qout[q] : q * A.ostride;")
+        w(ind + "((long long *)h)[6] = A.qout ? A.qout[q] : q * A.ostride;")
     else:
-        w(ind + "    ((long long *)h)[6] = wi.obase + A.ket.col[(long long)wi.tile * SIMINT_TILE + q] * A.stride;")
-    w(ind + "}")
+        w(ind + "((long long *)h)[6] = wi.obase + A.ket.col[(long long)wi.tile * SIMINT_TILE + q] * A.stride;")
     w("            }")
+    if p.G > 1:
+        w("            if (screen && tid == 0) ((unsigned *)qi)[14] = alive;   // read by the others behind the barrier")
 
 
 def _emit_vrr(p, w, part):

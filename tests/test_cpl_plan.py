@@ -148,3 +148,30 @@ def test_deep_plans_share_the_tops_in_another_way():
                 while sum(f):
                     assert f in nodes
                     f = step(f, mk_dir(f), -1)
+
+
+def test_screened_primitive_quartets_are_left_out():
+    """The bits of the mask the primitive loop tests are those of the lanes
+    that prepared that primitive quartet for the group's quartets, for every
+    batch shape of every plan; and the emitted loops test them."""
+    for am in CLASSES:
+        for p in (hip_cpl.plan(am, hip_cpl.base_G(am)), hip_cpl.split_plan(am), hip_cpl.deep_plan(am)):
+            if p is None:
+                continue
+            assert p.ent <= 16
+            for PBK in range(1, p.ent // p.NQ + 1):
+                every = sum(1 << (v * PBK) for v in range(p.NQ))
+                GB = p.ent // p.NQ // PBK
+                seen = set()
+                for gi in range(GB):
+                    for pp in range(PBK):
+                        bits = {b for b in range(32) if every << (gi * p.NQ * PBK + pp) >> b & 1}
+                        # block ((gi NQ + w) PBK + pp) is lane's, as the recurrence reads it
+                        assert bits == {(gi * p.NQ + w) * PBK + pp for w in range(p.NQ)}
+                        seen |= bits
+                assert seen == set(range(GB * p.NQ * PBK))
+    for am in [(1, 1, 1, 0), (2, 2, 2, 2), (3, 2, 3, 3)]:
+        text = hip_cpl.emit_cpl(am)
+        loops = text.split("for (int pp = 0; pp < npb_; ++pp) {\n")[1:]
+        assert loops and all(
+            x.lstrip().startswith("if (((alive >> (gi * NQ * PBK + pp)) & every) == 0) continue;") for x in loops)
