@@ -242,13 +242,20 @@ const char *simint_hip_last_error(void);
  * classes run the component-lane kernel where it is built, in FP64 also for
  * precision 1.  The values are family 1's bit for bit, except that without
  * HRR the primitive quartets are summed in up to eight parts: there they can
- * differ in the last places between launches of few and of many items. */
+ * differ in the last places between launches of few and of many items.
+ * The choice built in gives way to another family in two places, which setting
+ * a family (also the one returned) ends: (dp|dp) and (dd|pp) launches of 1024
+ * items and more of 16 primitive quartets and more run family 5, and lists
+ * of quartets of even depth run family 1 in place of 7 from a number of
+ * primitive quartets on, per class.  simint_hip_reset_class_kernels returns
+ * every class to what was built in. */
 int simint_hip_class_kernel(int la, int lb, int lc, int ld);
 int simint_hip_set_class_kernel(int la, int lb, int lc, int ld, int family);
 /* The same for the quartet-list calls: 1 = lane-per-quartet, 2 = wave-per-quartet,
  * 7 = component-lane. */
 int simint_hip_class_list_kernel(int la, int lb, int lc, int ld);
 int simint_hip_set_class_list_kernel(int la, int lb, int lc, int ld, int family);
+void simint_hip_reset_class_kernels(void);
 
 #ifdef __cplusplus
 }

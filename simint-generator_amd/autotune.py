@@ -10,11 +10,13 @@ pairs of depth 1-3 in an 8-bohr cube), and writes the fastest family per class t
 build to set each class's default):
 
     python simint-generator_amd/autotune.py [--natom 16] [--reps 3] [--out PATH]
-    python simint-generator_amd/autotune.py --list [--split]   # quartet-list kernels
+    python simint-generator_amd/autotune.py --list [--split] [--even]   # quartet-list kernels
 
 --list --split also times the lanes per quartet of the lane-per-quartet
 list launches per class and records the counts that beat the automatic
-choice ("list_split"; batch.QuartetBatch applies them).
+choice ("list_split"; batch.QuartetBatch applies them).  --list --even times
+lists of one depth and records from how many primitive quartets on the
+lane-per-quartet kernel beats the component-lane one ("list_even").
 """
 import argparse
 import json
@@ -38,11 +40,16 @@ def main():
     ap.add_argument("--split", action="store_true",
                     help="with --list: also time 1-16 lanes per quartet for the classes whose list kernel is "
                          "lane-per-quartet (merges 'list_split' into the output file)")
+    ap.add_argument("--even", action="store_true",
+                    help="with --list: also time lists of one depth in the classes whose list kernel is "
+                         "component-lane (merges 'list_even' into the output file)")
     a = ap.parse_args()
     if a.list:
         tune_lists(a)
         if a.split:
             tune_split(a)
+        if a.even:
+            tune_even(a)
         return None
     import torch
     import quartets
@@ -253,6 +260,77 @@ def tune_split(a):
     with open(a.out, "w") as f:
         json.dump(doc, f, indent=1, sort_keys=True)
     print("wrote", a.out, "(%d classes with a fixed lane count)" % len(split))
+
+
+def tune_even(a):
+    """Lists of 50 to 12800 quartets of one depth: for every class whose list
+    kernel (after the family tuning) is component-lane, the number of primitive
+    quartets from which the lane-per-quartet kernel is taken, below 16 primitive
+    quartets a quartet (timed at 1, the longest list only) and from there on
+    (timed at 16 and 256; the number that makes the timings' product least)."""
+    import itertools
+    import math
+    import numpy as np
+    import torch
+    import quartets
+    import simint
+    L = simint.lib()
+    if os.path.exists(a.out):
+        simint.apply_tuning(a.out)
+    lens = (50, 200, 800, 3200, 12800)
+    rng = np.random.default_rng(0)
+    sets = {}
+    for la, lb, depth in itertools.product(range(4), range(4), (1, 2, 4)):
+        shells = [(l, tuple(rng.uniform(0, 4, 3)), list(np.exp(rng.uniform(np.log(0.1), np.log(20), depth))),
+                   list(rng.uniform(0.1, 1.0, depth))) for _ in range(64) for l in (la, lb)]
+        basis = simint.Basis(shells)
+        hp = simint.Pairs.from_pairs(basis, [(2 * k, 2 * k + 1) for k in range(64)])
+        sets[la, lb, depth] = simint.DevicePairs(hp)
+        hp.free()
+        basis.free()
+    index = [torch.from_numpy(rng.integers(0, 64, lens[-1]).astype(np.int32)).cuda() for _ in range(2)]
+    out = torch.empty(lens[-1] * 10000, dtype=torch.float64, device="cuda")
+    stream = torch.cuda.ExternalStream(L.simint_hip_stream())
+
+    def ms(P, Q, n):
+        best = None
+        for rep in range(a.reps + 1):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record(stream)
+            simint.compute_list(P, Q, n, index[0].data_ptr(), index[1].data_ptr(), 0, out.data_ptr())
+            e1.record(stream)
+            simint.synchronize()
+            t = e0.elapsed_time(e1)
+            if rep > 0:
+                best = t if best is None else min(best, t)
+        return best
+    even = {}
+    for cls in itertools.product(range(4), repeat=4):
+        if L.simint_hip_class_list_kernel(*cls) != 7 or L.simint_hip_set_class_list_kernel(*cls, 1) < 0:
+            continue
+        t = {}
+        for fam in (1, 7):
+            L.simint_hip_set_class_list_kernel(*cls, fam)
+            for depth, n in [(1, lens[-1])] + [(d, n) for d in (2, 4) for n in lens]:
+                t[fam, depth, n] = ms(sets[cls[0], cls[1], depth], sets[cls[2], cls[3], depth], n)
+
+        def cost(line):
+            return sum(math.log(t[1 if n * d ** 4 >= line else 7, d, n]) for d in (2, 4) for n in lens)
+        never = 1 << 40
+        deep = min([never] + sorted({n * d ** 4 for d in (2, 4) for n in lens}, reverse=True), key=cost)
+        shallow = lens[-1] if t[1, 1, lens[-1]] < 0.97 * t[7, 1, lens[-1]] else 0
+        if deep < never or shallow:
+            name = quartets.simint_class_name(cls)
+            even[name] = [shallow, deep if deep < never else 0]
+            print("%-8s %s" % (name, even[name]), flush=True)
+    L.simint_hip_reset_class_kernels()
+    for d in sets.values():
+        d.free()
+    doc = json.load(open(a.out)) if os.path.exists(a.out) else {}
+    doc["list_even"] = even
+    with open(a.out, "w") as f:
+        json.dump(doc, f, indent=1, sort_keys=True)
+    print("wrote", a.out, "(%d classes)" % len(even))
 
 
 if __name__ == "__main__":

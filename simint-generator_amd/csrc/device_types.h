@@ -72,7 +72,8 @@ struct EriListArgs {
     const double *boys_grid;
     double tol2;
     double ket_screen_max;
-    int split;                 // lanes per quartet (1, 2, 4, 8) of the lane-per-quartet list kernels
+    int split;                 // lanes per quartet (a power of two up to 64) of the lane-per-quartet list kernels
+    long long depth = 0;       // most primitive quartets of a quartet (0: unknown)
 };
 
 struct EriArgs {
@@ -86,4 +87,5 @@ struct EriArgs {
     double ket_screen_max;         // simint_multi_shellpair.screen_max of the ket set
     long long stride;              // doubles per quartet in the output
     double *scratch;               // per-work-item staging (split kernels only)
+    long long depth = 0;           // most primitive quartets of a quartet (0: unknown)
 };

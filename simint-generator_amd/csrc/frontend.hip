@@ -398,6 +398,8 @@ int simint_hip_pairs_from_shells(const simint_hip_shells *S, int npair, const in
     p->screen_max = 1.e99;
     p->dev = d;
     p->bytes = bytes;
+    for (int k = 0; k < npair; k++) p->maxnp = std::max(p->maxnp, ppoff[k + 1] - ppoff[k]);
+    p->meannp = npair > 0 ? (double)ppoff[npair] / npair : 0.0;
     PairsLinear &lin = p->lin;
     lin.alpha = f.alpha_; lin.inv_alpha = f.inv; lin.prefac = f.prefac;
     lin.x = f.x; lin.y = f.y; lin.z = f.z;

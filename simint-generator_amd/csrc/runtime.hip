@@ -1076,8 +1076,16 @@ int simint_compute_ostei_deriv(int deriv, const simint_multi_shellpair *P, const
     memcpy(c.stage.p, im.buf.data(), im.buf.size());
     if ((e = copy_in(c, im.buf.size())) != hipSuccess) { set_err("copy to the device", e); return SIMINT_ERROR_HIP; }
 
+    long long most_p = 0, most_q = 0;   // primitives of a pair
+    for (int k = 0; k < nP; k++) most_p = std::max<long long>(most_p, P->nprim12[k]);
+    for (int k = 0; k < nQ; k++) most_q = std::max<long long>(most_q, Q->nprim12[k]);
+    const long long depth = most_p * most_q;
     size_t nst = 0;
-    for (auto &t : terms) nst = std::max(nst, (size_t)simint_dispatch_staging(t.am[0], t.am[1], t.am[2], t.am[3]));
+    for (auto &t : terms) {
+        const int family = simint_range_family(t.am[0], t.am[1], t.am[2], t.am[3], nit, depth);
+        t.fn = simint_family_launch(family, t.am[0], t.am[1], t.am[2], t.am[3]);
+        nst = std::max(nst, (size_t)simint_family_staging(family, t.am[0], t.am[1], t.am[2], t.am[3]));
+    }
     if (nst && (e = c.split.reserve(sizeof(double) * nst * SIMINT_TILE * (size_t)nit)) != hipSuccess) {
         set_err("hipMalloc", e);
         hipStreamSynchronize(c.s);   // the copy out of c.stage
@@ -1097,6 +1105,7 @@ int simint_compute_ostei_deriv(int deriv, const simint_multi_shellpair *P, const
         if (t.weight && t.centre == 3) a.ket.prefac = reinterpret_cast<const double *>(base + to.prefac_b2);
         a.items = reinterpret_cast<const WorkItem *>(base + items_off[k]);
         a.nitems = nit;
+        a.depth = depth;
         a.out = dout + t.off;
         a.boys_grid = g_dev.boys;
         a.tol2 = (screen_tol > 0.0 && P->screen && Q->screen) ? tol2 : 0.0;
@@ -1189,6 +1198,10 @@ int simint_hip_pairs_create(const simint_multi_shellpair *P, simint_hip_pairs **
     p->has_screen = P->screen != nullptr;
     p->dev = d;
     p->bytes = im.buf.size();
+    for (int k = 0; k < n; k++) {
+        p->maxnp = std::max(p->maxnp, P->nprim12[k]);
+        p->meannp += (double)P->nprim12[k] / n;
+    }
     p->lin = linear_ptrs(static_cast<char *>(d), lo);
     p->til = tiled_ptrs(static_cast<char *>(d), to);
     p->ntile = to.ntile;
@@ -1276,6 +1289,7 @@ struct RangeTerm {
     int am[4];
     simint_launch_fn fn;
     int weight;   // -1: none
+    bool fp32 = false;   // fn is the FP32-VRR launcher
 };
 
 // items_out / nitems_out / tstart_out (optional): the work items of the first
@@ -1311,10 +1325,18 @@ long long range_launch(const simint_hip_pairs *P, const simint_hip_pairs *Q, int
     }
     if ((e = c.range_enter()) != hipSuccess) { set_err("hipStreamWaitEvent", e); return SIMINT_ERROR_HIP; }
     const RangeDone done{c};
+    const long long depth = (long long)P->maxnp * Q->maxnp;
     size_t nst = 0;
-    for (int t = 0; t < nterm; t++)
-        nst = std::max(nst, (size_t)simint_dispatch_staging(terms[t].am[0], terms[t].am[1], terms[t].am[2],
-                                                            terms[t].am[3]));
+    simint_launch_fn fn[kMaxTerms];
+    bool stages[kMaxTerms];
+    for (int t = 0; t < nterm; t++) {
+        const int *am = terms[t].am;
+        const int family = simint_range_family(am[0], am[1], am[2], am[3], nitems, depth);
+        const size_t n = terms[t].fp32 ? 0 : (size_t)simint_family_staging(family, am[0], am[1], am[2], am[3]);
+        fn[t] = terms[t].fp32 ? terms[t].fn : simint_family_launch(family, am[0], am[1], am[2], am[3]);
+        stages[t] = n > 0;
+        nst = std::max(nst, n);
+    }
     const size_t items_bytes = sizeof(WorkItem) * (size_t)nitems * nterm;
     if ((e = c.grow(c.items, items_bytes + sizeof(long long) * (size_t)nbra)) != hipSuccess ||
         (e = c.grow(c.split, sizeof(double) * nst * SIMINT_TILE * (size_t)nitems)) != hipSuccess) {
@@ -1376,9 +1398,8 @@ long long range_launch(const simint_hip_pairs *P, const simint_hip_pairs *Q, int
         }
         std::sort(order, order + nterm, [&](int a, int b) { return cost[a] > cost[b]; });
         for (int k = 0; k < nterm; k++) {
-            const RangeTerm &T = terms[order[k]];
             // kernels that stage share c.split: one after another
-            if (!simint_dispatch_staging(T.am[0], T.am[1], T.am[2], T.am[3]))
+            if (!stages[order[k]])
                 on[order[k]] = (int)(std::min_element(load, load + ThreadCtx::kSide + 1) - load);
             load[on[order[k]]] += cost[order[k]];
             used[on[order[k]]] = true;
@@ -1401,12 +1422,13 @@ long long range_launch(const simint_hip_pairs *P, const simint_hip_pairs *Q, int
         if (T.weight == 3) a.ket.prefac = Q->twb;
         a.items = x.items + nitems * t;
         a.nitems = nitems;
+        a.depth = depth;
         a.out = d_outs[t];
         a.boys_grid = g_dev.boys;
         a.tol2 = (screen_tol > 0.0 && P->has_screen && Q->has_screen) ? screen_tol * screen_tol : 0.0;
         a.ket_screen_max = Q->screen_max;
         a.stride = x.stride[t];
-        failed = T.fn(&a, on[t] ? side[on[t] - 1] : c.s);
+        failed = fn[t](&a, on[t] ? side[on[t] - 1] : c.s);
     }
     for (int k = 0; k < ThreadCtx::kSide; k++) {
         if (!used[k + 1]) continue;
@@ -1436,6 +1458,7 @@ long long simint_hip_compute_eri_range(const simint_hip_pairs *P, const simint_h
     if (!ensure_device()) return SIMINT_ERROR_NO_DEVICE;
     RangeTerm t{{P->am1, P->am2, Q->am1, Q->am2}, nullptr, -1};
     if (precision == 1) t.fn = simint_dispatch_mixed(P->am1, P->am2, Q->am1, Q->am2);
+    t.fp32 = t.fn != nullptr;
     if (!t.fn) t.fn = simint_dispatch(P->am1, P->am2, Q->am1, Q->am2);
     if (!t.fn) { t_err = "class not built"; return SIMINT_ERROR_UNSUPPORTED; }
     return range_launch(P, Q, b0, nbra, ket_lo, ket_hi, &out_off, &t, 1, screen_tol, &d_out);
@@ -1451,6 +1474,7 @@ long long simint_hip_compute_jk_range(const simint_hip_pairs *P, const simint_hi
     if (!ensure_device()) return SIMINT_ERROR_NO_DEVICE;
     RangeTerm t{{P->am1, P->am2, Q->am1, Q->am2}, nullptr, -1};
     if (precision == 1) t.fn = simint_dispatch_mixed(P->am1, P->am2, Q->am1, Q->am2);
+    t.fp32 = t.fn != nullptr;
     if (!t.fn) t.fn = simint_dispatch(P->am1, P->am2, Q->am1, Q->am2);
     if (!t.fn) { t_err = "class not built"; return SIMINT_ERROR_UNSUPPORTED; }
     const WorkItem *items = nullptr;
@@ -1514,6 +1538,7 @@ long long simint_hip_compute_eri_diag(const simint_hip_pairs *P, double *d_out)
     a.ket = P->til;
     a.items = static_cast<const WorkItem *>(c.items.p);
     a.nitems = P->n;
+    a.depth = (long long)P->maxnp * P->maxnp;
     a.out = d_out;
     a.boys_grid = g_dev.boys;
     a.tol2 = 0.0;
@@ -1579,22 +1604,39 @@ EriListArgs list_args(const simint_hip_pairs *P, const simint_hip_pairs *Q, long
     a.tol2 = (screen_tol > 0.0 && P->has_screen && Q->has_screen) ? screen_tol * screen_tol : 0.0;
     a.ket_screen_max = Q->screen_max;
     a.split = 1;
+    a.depth = (long long)P->maxnp * Q->maxnp;
     return a;
 }
 
 thread_local int t_list_split = 0;   // 0: by list length
 
+// Launcher of a list of n quartets of one class over these pairs.  A list is
+// taken to be of even depth if the pairs' mean depths multiply to half their
+// largest or more: a wavefront's lanes then run equally long.
+simint_list_launch_fn list_launch(const simint_hip_pairs *P, const simint_hip_pairs *Q, int la, int lb, int lc, int ld,
+                                  long long n)
+{
+    const long long depth = (long long)P->maxnp * Q->maxnp;
+    if (2.0 * P->meannp * Q->meannp >= (double)depth) {
+        const simint_list_launch_fn fn = simint_dispatch_list_even(la, lb, lc, ld, n, depth);
+        if (fn) return fn;
+    }
+    return simint_dispatch_list(la, lb, lc, ld);
+}
+
 // Lanes per quartet for a lane-per-quartet list launch of n quartets: enough
 // that the launch has about 65536 lanes (a short list of one class otherwise
 // occupies a few dozen wavefronts), up to 16; up to a whole wavefront while
 // it has fewer than 16384 (a list of six quartets of up to 1296 primitive
-// quartets otherwise leaves 81 of them to one lane).
-int list_split(long long n)
+// quartets otherwise leaves 81 of them to one lane) and a quartet has as many
+// primitive quartets: 50 uncontracted (pp|pp) quartets take 9.7 us with 16
+// lanes each and 11.7 with 64.
+int list_split(long long n, long long depth)
 {
     if (t_list_split > 0) return t_list_split;
     int s = 1;
     while (s < 16 && n * s < 65536) s *= 2;
-    while (s < 64 && n * s < 16384) s *= 2;
+    while (s < 64 && n * s < 16384 && s < depth) s *= 2;
     return s;
 }
 
@@ -1608,14 +1650,14 @@ long long simint_hip_compute_eri_list(const simint_hip_pairs *P, const simint_hi
 {
     if (!P || !Q || nquartet < 0 || (nquartet > 0 && (!d_qbra || !d_qket || !d_out))) return SIMINT_ERROR_ARGUMENT;
     if (!ensure_device()) return SIMINT_ERROR_NO_DEVICE;
-    const simint_list_launch_fn fn = simint_dispatch_list(P->am1, P->am2, Q->am1, Q->am2);
+    const simint_list_launch_fn fn = list_launch(P, Q, P->am1, P->am2, Q->am1, Q->am2, nquartet);
     if (!fn) { t_err = "class not built"; return SIMINT_ERROR_UNSUPPORTED; }
     if (nquartet == 0) return 0;
     EriListArgs a = list_args(P, Q, nquartet, d_qbra, d_qket, screen_tol);
     a.qout = d_qout;
     a.ostride = (long long)ncart(P->am1) * ncart(P->am2) * ncart(Q->am1) * ncart(Q->am2);
     a.out = d_out;
-    a.split = list_split(nquartet);
+    a.split = list_split(nquartet, a.depth);
     hipError_t e = fn(&a, ctx().s);
     if (e != hipSuccess) { set_err("class kernel launch", e); return SIMINT_ERROR_HIP; }
     return nquartet;
@@ -1674,7 +1716,7 @@ long long deriv1_list(const simint_hip_pairs *P, const simint_hip_pairs *Q, long
         // several lanes a quartet add its primitive quartets in another order,
         // which the HRR and the weight 2a amplify: only where the HRR transfers
         // one unit of AM at most (six (sd|pp) quartets on a lane each took 1.2 ms)
-        if (std::min(t.am[0], t.am[1]) + std::min(t.am[2], t.am[3]) <= 1) a.split = list_split(nquartet);
+        if (std::min(t.am[0], t.am[1]) + std::min(t.am[2], t.am[3]) <= 1) a.split = list_split(nquartet, a.depth);
         if ((e = fns[k](&a, c.s)) != hipSuccess) { set_err("class kernel launch", e); return SIMINT_ERROR_HIP; }
         if (t.sign > 0) d.plus[t.centre] = a.out;
         else d.minus[t.centre] = a.out;

@@ -22,6 +22,8 @@ struct simint_hip_pairs {
     PairsTiled til;
     int ntile;
     size_t bytes = 0;                            // device memory held
+    int maxnp = 0;                               // primitives of a pair: the most,
+    double meannp = 0.0;                         // and the mean
     const double *wa = nullptr, *wb = nullptr;   // linear prefac * alpha2, prefac * beta2
     const double *twa = nullptr, *twb = nullptr; // the same in the tiled view
 };

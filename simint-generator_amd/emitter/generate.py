@@ -131,7 +131,8 @@ def mixed_candidate(am):
     return max(am) <= MIXED_MAXAM
 
 
-def dispatch_text(maxam, lpq, wpq, selection, lpqs=None, list_selection=None, lpqsf=None, cpl=()):
+def dispatch_text(maxam, lpq, wpq, selection, lpqs=None, list_selection=None, lpqsf=None, cpl=(), deep=None,
+                  even=None):
     # tables reach one AM above the maximum when derivative terms are built
     n = 1 + max(max(am) for am in wpq)
     lines = ["// Generated by simint-generator_amd/emitter/generate.py -- do not edit.",
@@ -217,23 +218,35 @@ def dispatch_text(maxam, lpq, wpq, selection, lpqs=None, list_selection=None, lp
     table("g_wpql", set(wpq), "wpql", "simint_list_launch_fn")
     table("g_cpl", set(cpl), "cpl")
     table("g_cpll", set(cpl), "cpll", "simint_list_launch_fn")
+    # the built-in choice carries BUILTIN: only it gives way to another family
+    # by the size of a launch
+    lines.append("constexpr int BUILTIN = 16, FAMILY = 15;")
     flat = []
     for am in itertools.product(range(n), repeat=4):
-        flat.append(str(selection.get(am, 0)))
+        flat.append("%d" % (selection[am] | 16) if am in selection else "0")
     lines.append("std::atomic<int> g_sel[N * N * N * N] = {" + ", ".join(flat) + "};")
+    lines.append("const int g_sel_built[N * N * N * N] = {" + ", ".join(flat) + "};")
     flat = []
     for am in itertools.product(range(n), repeat=4):
-        flat.append(str((list_selection or {}).get(am, 2)))
+        flat.append("%d" % ((list_selection or {}).get(am, 2) | 16))
     lines.append("std::atomic<int> g_sel_list[N * N * N * N] = {" + ", ".join(flat) + "};")
+    lines.append("const int g_sel_list_built[N * N * N * N] = {" + ", ".join(flat) + "};")
+    lines.append("const unsigned char g_deep[N * N * N * N] = {"
+                 + ", ".join(str((deep or {}).get(am, 0)) for am in itertools.product(range(n), repeat=4)) + "};")
+    lines.append("// primitive quartets from which a list of even depth runs the lane-per-quartet kernel: of")
+    lines.append("// quartets of fewer than EVEN_DEPTH, and of deeper ones (0: never)")
+    lines.append("constexpr int EVEN_DEPTH = %d;" % EVEN_DEPTH)
+    lines.append("const int g_even[N * N * N * N][2] = {"
+                 + ", ".join("{%d, %d}" % tuple((even or {}).get(am, (0, 0)))
+                             for am in itertools.product(range(n), repeat=4)) + "};")
     lines.append("inline int idx(int a, int b, int c, int d) { return ((a * N + b) * N + c) * N + d; }")
     lines.append("inline bool in_range(int a, int b, int c, int d)")
     lines.append("{ return a >= 0 && b >= 0 && c >= 0 && d >= 0 && a < N && b < N && c < N && d < N; }")
     lines.append("}  // namespace")
     lines.append("")
-    lines.append("simint_launch_fn simint_dispatch(int la, int lb, int lc, int ld)")
+    lines.append("simint_launch_fn simint_family_launch(int s, int la, int lb, int lc, int ld)")
     lines.append("{")
     lines.append("    if (!in_range(la, lb, lc, ld)) return nullptr;")
-    lines.append("    const int s = g_sel[idx(la, lb, lc, ld)].load(std::memory_order_relaxed);")
     lines.append("    if (s == 1) return g_lpq[la][lb][lc][ld];")
     lines.append("    if (s == 2) return g_wpq[la][lb][lc][ld];")
     lines.append("    if (s == 3) return g_lpqs_a[la][lb][lc][ld];")
@@ -244,34 +257,57 @@ def dispatch_text(maxam, lpq, wpq, selection, lpqs=None, list_selection=None, lp
     lines.append("    return nullptr;")
     lines.append("}")
     lines.append("")
-    lines.append("int simint_dispatch_staging(int la, int lb, int lc, int ld)")
+    lines.append("int simint_family_staging(int s, int la, int lb, int lc, int ld)")
     lines.append("{")
     lines.append("    if (!in_range(la, lb, lc, ld)) return 0;")
-    lines.append("    const int s = g_sel[idx(la, lb, lc, ld)].load(std::memory_order_relaxed);")
     lines.append("    if (s == 5 || s == 6) return g_stage_f[la][lb][lc][ld];")
     lines.append("    return (s == 3 || s == 4) ? g_stage[la][lb][lc][ld] : 0;")
     lines.append("}")
     lines.append("")
+    lines.append("int simint_range_family(int la, int lb, int lc, int ld, long long items, long long depth)")
+    lines.append("{")
+    lines.append("    if (!in_range(la, lb, lc, ld)) return 0;")
+    lines.append("    const int i = idx(la, lb, lc, ld);")
+    lines.append("    const int s = g_sel[i].load(std::memory_order_relaxed);")
+    lines.append("    if ((s & BUILTIN) && g_deep[i] && items >= %d && depth >= %d) return g_deep[i];" % (DEEP_ITEMS, DEEP_DEPTH))
+    lines.append("    return s & FAMILY;")
+    lines.append("}")
+    lines.append("")
+    lines.append("simint_launch_fn simint_dispatch(int la, int lb, int lc, int ld)")
+    lines.append("{ return simint_family_launch(simint_range_family(la, lb, lc, ld, 0, 0), la, lb, lc, ld); }")
+    lines.append("")
+    lines.append("int simint_dispatch_staging(int la, int lb, int lc, int ld)")
+    lines.append("{ return simint_family_staging(simint_range_family(la, lb, lc, ld, 0, 0), la, lb, lc, ld); }")
+    lines.append("")
     lines.append("simint_launch_fn simint_dispatch_mixed(int la, int lb, int lc, int ld)")
     lines.append("{")
     lines.append("    if (!in_range(la, lb, lc, ld)) return nullptr;")
-    lines.append("    const int s = g_sel[idx(la, lb, lc, ld)].load(std::memory_order_relaxed);")
+    lines.append("    const int s = g_sel[idx(la, lb, lc, ld)].load(std::memory_order_relaxed) & FAMILY;")
     lines.append("    return s == 1 ? g_lpqm[la][lb][lc][ld] : nullptr;")
     lines.append("}")
     lines.append("")
     lines.append("simint_list_launch_fn simint_dispatch_list(int la, int lb, int lc, int ld)")
     lines.append("{")
     lines.append("    if (!in_range(la, lb, lc, ld)) return nullptr;")
-    lines.append("    const int s = g_sel_list[idx(la, lb, lc, ld)].load(std::memory_order_relaxed);")
+    lines.append("    const int s = g_sel_list[idx(la, lb, lc, ld)].load(std::memory_order_relaxed) & FAMILY;")
     lines.append("    if (s == 1 && g_lpql[la][lb][lc][ld]) return g_lpql[la][lb][lc][ld];")
     lines.append("    if (s == 7 && g_cpll[la][lb][lc][ld]) return g_cpll[la][lb][lc][ld];")
     lines.append("    return g_wpql[la][lb][lc][ld];")
     lines.append("}")
     lines.append("")
+    lines.append("simint_list_launch_fn simint_dispatch_list_even(int la, int lb, int lc, int ld, long long n, long long depth)")
+    lines.append("{")
+    lines.append("    if (!in_range(la, lb, lc, ld)) return nullptr;")
+    lines.append("    const int i = idx(la, lb, lc, ld);")
+    lines.append("    const int from = g_even[i][depth >= EVEN_DEPTH];")
+    lines.append("    if (g_sel_list[i].load(std::memory_order_relaxed) != (7 | BUILTIN) || from == 0 || n * depth < from) return nullptr;")
+    lines.append("    return g_lpql[la][lb][lc][ld];")
+    lines.append("}")
+    lines.append("")
     lines.append('extern "C" int simint_hip_class_list_kernel(int la, int lb, int lc, int ld)')
     lines.append("{")
     lines.append("    if (!in_range(la, lb, lc, ld)) return 0;")
-    lines.append("    return g_sel_list[idx(la, lb, lc, ld)].load();")
+    lines.append("    return g_sel_list[idx(la, lb, lc, ld)].load() & FAMILY;")
     lines.append("}")
     lines.append("")
     lines.append('extern "C" int simint_hip_set_class_list_kernel(int la, int lb, int lc, int ld, int family)')
@@ -281,13 +317,13 @@ def dispatch_text(maxam, lpq, wpq, selection, lpqs=None, list_selection=None, lp
     lines.append("    if (family == 2 && !g_wpql[la][lb][lc][ld]) return -1;")
     lines.append("    if (family == 7 && !g_cpll[la][lb][lc][ld]) return -1;")
     lines.append("    if (family != 1 && family != 2 && family != 7) return -1;")
-    lines.append("    return g_sel_list[idx(la, lb, lc, ld)].exchange(family);")
+    lines.append("    return g_sel_list[idx(la, lb, lc, ld)].exchange(family) & FAMILY;")
     lines.append("}")
     lines.append("")
     lines.append('extern "C" int simint_hip_class_kernel(int la, int lb, int lc, int ld)')
     lines.append("{")
     lines.append("    if (!in_range(la, lb, lc, ld)) return 0;")
-    lines.append("    return g_sel[idx(la, lb, lc, ld)].load();")
+    lines.append("    return g_sel[idx(la, lb, lc, ld)].load() & FAMILY;")
     lines.append("}")
     lines.append("")
     lines.append('extern "C" int simint_hip_set_class_kernel(int la, int lb, int lc, int ld, int family)')
@@ -301,7 +337,15 @@ def dispatch_text(maxam, lpq, wpq, selection, lpqs=None, list_selection=None, lp
     lines.append("    if (family == 6 && !g_lpqs_d[la][lb][lc][ld]) return -1;")
     lines.append("    if (family == 7 && !g_cpl[la][lb][lc][ld]) return -1;")
     lines.append("    if (family < 1 || family > 7) return -1;")
-    lines.append("    return g_sel[idx(la, lb, lc, ld)].exchange(family);")
+    lines.append("    return g_sel[idx(la, lb, lc, ld)].exchange(family) & FAMILY;")
+    lines.append("}")
+    lines.append("")
+    lines.append('extern "C" void simint_hip_reset_class_kernels(void)')
+    lines.append("{")
+    lines.append("    for (int i = 0; i < N * N * N * N; i++) {")
+    lines.append("        g_sel[i] = g_sel_built[i];")
+    lines.append("        g_sel_list[i] = g_sel_list_built[i];")
+    lines.append("    }")
     lines.append("}")
     return "\n".join(lines) + "\n"
 
@@ -309,16 +353,35 @@ def dispatch_text(maxam, lpq, wpq, selection, lpqs=None, list_selection=None, lp
 FAMILIES = {"lpq": 1, "wpq": 2, "lpqs_a": 3, "lpqs_b": 4, "lpqsf_a": 5, "lpqsf_b": 6, "cpl": 7}
 
 
-def load_tuning(pkg_root, key="family"):
-    """Tuned family per class from tuning.json ("family": prefix kernels,
-    "list_family": quartet-list kernels)."""
+# The component-lane kernels spread one quartet over lanes; many deep quartets
+# run faster where staging keeps every lane busy.  "deep_family" of tuning.json
+# names the family of a class for launches of at least DEEP_ITEMS work items of
+# DEEP_DEPTH primitive quartets: 4096 items of (dd|pp) take 1.57 ms in the
+# component-lane kernel and 1.25 ms in the split one at 16 primitive quartets,
+# 6.9 and 4.7 ms at 81; of (dp|dp) 1.37 and 1.23, 6.1 and 4.7 ms; at one
+# primitive quartet 0.28 and 0.58 ms; 256 items of 81 0.55 and 1.15 ms.
+DEEP_ITEMS = 1024
+DEEP_DEPTH = 16
+# Lists tuned to the component-lane kernels on a stream of mixed depths, whose
+# lane-per-quartet wavefronts wait for their deepest lane: a list of even depth
+# runs the lane-per-quartet kernel from "list_even" of tuning.json primitive
+# quartets on (below EVEN_DEPTH a quartet, and from there; autotune.py --list
+# --even).  3200 (fp|ps) quartets of 16 primitive quartets: 84 us in the
+# component-lane kernels (38 unshared), 15 us in the other.
+EVEN_DEPTH = 16
+
+
+def load_tuning(pkg_root, key="family", names=FAMILIES):
+    """Tuned value per class from tuning.json ("family": prefix kernels,
+    "list_family": quartet-list kernels, "deep_family", "list_even"); names
+    maps it to a number (None: as it is)."""
     path = os.path.join(pkg_root, "tuning.json")
     if not os.path.exists(path):
         return {}
     d = json.load(open(path))
     out = {}
     for name, fam in d.get(key, {}).items():
-        out[tuple("spdfghik".index(c) for c in name.split("_"))] = FAMILIES[fam]
+        out[tuple("spdfghik".index(c) for c in name.split("_"))] = names[fam] if names else fam
     return out
 
 
@@ -390,7 +453,10 @@ def generate(pkg_root, include_root, maxam, lpq_ok=None):
             list_sel[am] = 2
     for am in gterms:
         list_sel[am] = selection[am]
-    _write(os.path.join(gen, "dispatch.cpp"), dispatch_text(maxam, lpq, wpq, selection, lpqs, list_sel, lpqsf, cpl))
+    deep = {am: f for am, f in load_tuning(pkg_root, "deep_family").items() if built(am, f) and am in selection}
+    even = {am: t for am, t in load_tuning(pkg_root, "list_even", None).items() if am in lpq and am in cpl}
+    _write(os.path.join(gen, "dispatch.cpp"), dispatch_text(maxam, lpq, wpq, selection, lpqs, list_sel, lpqsf, cpl,
+                                                        deep, even))
     fname = {v: k for k, v in FAMILIES.items()}
     info = {hip_lpq.class_name(am): dict(class_info(am), kernel=fname[selection[am]], split_groups=lpqs.get(am, []),
                                          split_kernels=[hip_lpqs.kernel_name(am, G) for G in lpqs.get(am, [])],

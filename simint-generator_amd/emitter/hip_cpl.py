@@ -55,7 +55,19 @@ ENT = 16           # primitive quartets per setup batch (one lane each), at most
 QINFO = 8          # per quartet: AB and CD, output base
 LDS_CU = 160 * 1024
 AREA_GOOD = 22 * 1024    # HRR area up to which four to eight wavefronts share a CU
-SPLIT_GROUPS = 4096      # list launches of at most this many groups share a group
+# List launches of at most SPLIT_GROUPS groups share a group between wavefronts
+# where a quartet has SPLIT_DEEP primitive quartets or more, of SPLIT_SOME from
+# SPLIT_DEPTH on (SPLIT_GROUPS where the unshared kernel has one wavefront a
+# SIMD: 3200 (dd|dd) quartets of 16 take 146 us unshared and 137 shared, of
+# (fd|pp) 54 and 81), of SPLIT_FEW (one a compute unit) whatever the depth: for
+# one primitive quartet seven of eight wavefronts wait.  3200 (fp|ps) quartets
+# of 1, 16 and 256 primitive quartets: 11, 38 and 474 us unshared, 57, 84 and
+# 275 shared; 200: 10, 35 and 442, 7, 10 and 25.
+SPLIT_GROUPS = 4096
+SPLIT_SOME = 1024
+SPLIT_FEW = 256
+SPLIT_DEPTH = 16
+SPLIT_DEEP = 64
 SPLIT_W = 4              # between so many wavefronts (primitive quartets: up to twice as many)
 # Lists of at most this many groups (four classes side by side then have one
 # a compute unit) share a group's tops between twice as many wavefronts,
@@ -342,8 +354,9 @@ def emit_cpl(am):
     w('#include "../boys_device.h"')
     w("")
     w("namespace {")
-    w("constexpr int NE = %d, NPC = %d, QINFO = %d, SPLIT_GROUPS = %d, DEEP_GROUPS = %d;"
-      % (p.NE, p.npc, QINFO, SPLIT_GROUPS, DEEP_GROUPS))
+    w("constexpr int NE = %d, NPC = %d, QINFO = %d, DEEP_GROUPS = %d;" % (p.NE, p.npc, QINFO, DEEP_GROUPS))
+    w("constexpr int SPLIT_GROUPS = %d, SPLIT_SOME = %d, SPLIT_FEW = %d, SPLIT_DEPTH = %d, SPLIT_DEEP = %d;"
+      % (SPLIT_GROUPS, SPLIT_SOME if p.occ > 1 else SPLIT_GROUPS, SPLIT_FEW, SPLIT_DEPTH, SPLIT_DEEP))
     w("// per wide component: chain directions, chain exponents, exponents, lane distances to e - 1_d")
     w("__constant__ __attribute__((aligned(16))) unsigned int lane_tab[NE][4] = {")
     for r in p.lane_tables():
@@ -524,7 +537,8 @@ def _emit_launchers(p, ps, pd, w):
         w("        hipLaunchKernelGGL(eri_cpld_%s, dim3((unsigned)ng), dim3(64, %d), 0, s, *a, 1);" % (name, pd.W))
         w("        return hipGetLastError();")
         w("    }")
-    w("    if (ng <= SPLIT_GROUPS) {")
+    w("    const long long depth = a->depth > 0 ? a->depth : SPLIT_DEEP;")
+    w("    if (ng <= (depth >= SPLIT_DEEP ? SPLIT_GROUPS : depth >= SPLIT_DEPTH ? SPLIT_SOME : SPLIT_FEW)) {")
     w("        hipLaunchKernelGGL(eri_cpls_%s, dim3((unsigned)ng), dim3(64, %d), 0, s, *a, 1);" % (name, ps.W))
     w("        return hipGetLastError();")
     w("    }")

@@ -387,21 +387,35 @@ def emit_lpq(am, mixed=False):
     return w.text()
 
 
-# Small launches: several wavefronts share an item's primitive quartets while
-# the launch has fewer than SHARE_ITEMS wavefronts (the chip holds 4096), eight
-# at most.  A 12-atom molecule's (ss|ss) launches are a few dozen items of up
-# to 1296 primitive quartets: 82 us each with one wavefront an item, 24 us so.
-# Classes without HRR add the wavefronts' sums at the end.  An HRR amplifies
-# the rounding of another order of the sum, so the others keep the order:
+# Small launches: several wavefronts share an item's primitive quartets, eight
+# at most and no more than it has.  A 12-atom molecule's (ss|ss) launches are a
+# few dozen items of up to 1296 primitive quartets: 82 us each with one
+# wavefront an item, 24 us so.
+# Classes without HRR add the wavefronts' sums at the end, while the launch has
+# fewer than SHARE_ITEMS wavefronts (the chip holds 4096); of more than
+# SHARE_TOPS sums up to SHARE_ITEMS / 2, one for every SIMD, which such a
+# kernel's registers fill (1024 items of (fs|fs) take 369 us with one wavefront
+# each, 405 with two and 500 with four, 256 of them 343, 204 and 133).  An HRR
+# amplifies the rounding of another order of the sum, so the others keep it:
 #  * (ab|ss) and (ss|cd): the wavefronts take the primitive quartets in turn,
 #    leave the contracted terms in the local data share, and every contracted
-#    value is added up by one of them in the order one wavefront alone adds it;
-#  * the rest run the component-lane kernel up to SMALL_ITEMS items, which
-#    spreads a quartet over lanes instead and gives the same values: 81
-#    primitive quartets of (dp|ps) take 196 us with one wavefront an item and
-#    78 us so for 1 item, 202 and 128 us for 128, 201 and 224 for 256.
+#    value is added up by one of them in the order one wavefront alone adds it,
+#    where all items' terms fit the compute units' local data shares at once:
+#    256 items of 81 primitive quartets of (dd|ss) take 134 us with one
+#    wavefront and 84 with four, 1024 of them 140 and 317; two wavefronts are
+#    slower than one always;
+#  * the rest run the component-lane kernel, which spreads a quartet over lanes
+#    instead and gives the same values, up to LANE_ITEMS items and
+#    LANE_ITEMS_PER_DEPTH for each primitive quartet of the deepest: over the
+#    60 classes it takes 0.58, 0.70 and 0.86 of the time with 32, 64 and 128
+#    items of 16 primitive quartets, 0.76, 0.85 and 0.98 with 4, but 1.12, 1.21
+#    and 1.33 with 1.  Where the wide side has AM 2 in all a quartet is 10
+#    lanes' work and LANE_ITEMS_2 the line ((ps|pp): 0.97 with 32, 1.19 with 128).
 SHARE_ITEMS = 2048
-SMALL_ITEMS = 128
+SHARE_TOPS = 36
+LANE_ITEMS = 128
+LANE_ITEMS_2 = 32
+LANE_ITEMS_PER_DEPTH = 8
 SHARE_SUM = 8       # contracted values added per round at the end (classes without HRR)
 
 
@@ -413,7 +427,7 @@ def share_kind(am):
     if not g.bra_hrr_needed() and not g.ket_hrr_needed():
         return "sum" if len(g.top_keys) <= 128 else None
     if min(g.e_hi, g.f_hi) == 0:
-        return "turn" if len(g.top_keys) <= 64 else None
+        return "turn" if len(g.top_keys) <= 32 else None
     return "lanes" if hip_cpl.candidate(am) else None
 
 
@@ -435,16 +449,33 @@ def _emit_lpq_launcher(am, w, fp):
     w('extern "C" hipError_t simint_launch_%s(const EriArgs *a, hipStream_t s)' % kname)
     w("{")
     w("    if (a->nitems <= 0) return hipSuccess;")
+    if kind:
+        w("    const long long depth = a->depth > 0 ? a->depth : 4096;   // unknown: as deep ones")
     if kind == "lanes":
-        w("    if (a->nitems <= %d) return simint_launch_cpl_%s(a, s);" % (SMALL_ITEMS, class_name(am)))
-    elif kind:
+        g = graph(*am)
+        most_items = LANE_ITEMS_2 if max(g.e_hi, g.f_hi) == 2 else LANE_ITEMS
+        w("    if (a->nitems <= (%d * depth < %d ? %d * depth : %d)) return simint_launch_cpl_%s(a, s);"
+          % (LANE_ITEMS_PER_DEPTH, most_items, LANE_ITEMS_PER_DEPTH, most_items, class_name(am)))
+    elif kind == "sum":
         w("    int waves = 1;")
-        w("    while (waves < %d && a->nitems * waves < %d) waves *= 2;" % (most, SHARE_ITEMS))
+        room = ("a->nitems * waves < %d" % SHARE_ITEMS if len(graph(*am).top_keys) <= SHARE_TOPS
+                else "2 * a->nitems * waves <= %d" % (SHARE_ITEMS // 2))
+        w("    while (waves < %d && 2 * waves <= depth && %s) waves *= 2;" % (most, room))
         w("    if (waves > 1) {")
-        w("        hipLaunchKernelGGL(eri_%s, dim3((unsigned)a->nitems), dim3(64, waves), waves * %du, s, *a);"
-          % (kname.replace("_", "k_", 1), 2 * 512 * len(graph(*am).top_keys) if kind == "turn" else 0))
+        w("        hipLaunchKernelGGL(eri_%s, dim3((unsigned)a->nitems), dim3(64, waves), 0, s, *a);"
+          % kname.replace("_", "k_", 1))
         w("        return hipGetLastError();")
         w("    }")
+    elif kind == "turn":
+        terms = 2 * 512 * len(graph(*am).top_keys)   # of one wavefront, both buffers
+        for waves in (8, 4):
+            if waves <= most:
+                w("    if (a->nitems <= %d && depth >= %d%s) {"
+                  % (256 * (160 * 1024 // (waves * terms)), waves, "" if waves == most else " && depth < %d" % most))
+                w("        hipLaunchKernelGGL(eri_%s, dim3((unsigned)a->nitems), dim3(64, %d), %du, s, *a);"
+                  % (kname.replace("_", "k_", 1), waves, waves * terms))
+                w("        return hipGetLastError();")
+                w("    }")
     w("    hipLaunchKernelGGL(eri_%s, dim3((unsigned)a->nitems), dim3(64), 0, s, *a);" % kname)
     w("    return hipGetLastError();")
     w("}")
@@ -539,7 +570,7 @@ def _emit_lpq_prefix(am, w, fp, hrr_fp="double", shared=None):
         w("    const int i0 = ib0 + wave / jstep, j0 = wave % jstep;")
     if shared == "turn":
         w("    extern __shared__ double terms[];")
-        w("    constexpr int OWN = %d;   // values a wavefront adds up, with two of them or more" % ((ntop + 1) // 2))
+        w("    constexpr int OWN = %d;   // values a wavefront adds up, with four of them or more" % ((ntop + 3) // 4))
         w("    double own[OWN];")
         w("#pragma unroll")
         w("    for (int k = 0; k < OWN; ++k) own[k] = 0.0;")

@@ -56,6 +56,7 @@ EXPORTS = [
     "simint_hip_pairs_create", "simint_hip_pairs_free", "simint_hip_pairs_count",
     "simint_hip_compute_eri_prefix", "simint_hip_compute_eri_diag", "simint_hip_synchronize",
     "simint_hip_stream", "simint_hip_last_error", "simint_hip_class_kernel", "simint_hip_set_class_kernel",
+    "simint_hip_reset_class_kernels",
     "simint_hip_compute_eri_list", "simint_hip_compute_eri_range", "simint_hip_deriv1_worksize",
     "simint_hip_compute_eri_deriv1_range", "simint_hip_set_stream", "simint_hip_class_list_kernel",
     "simint_hip_set_list_split",
@@ -135,6 +136,8 @@ def lib():
         L.simint_hip_last_error.restype = ctypes.c_char_p
         L.simint_hip_class_kernel.argtypes = [c_int] * 4
         L.simint_hip_set_class_kernel.argtypes = [c_int] * 5
+        L.simint_hip_reset_class_kernels.argtypes = []
+        L.simint_hip_reset_class_kernels.restype = None
         L.simint_hip_class_list_kernel.argtypes = [c_int] * 4
         L.simint_hip_set_class_list_kernel.argtypes = [c_int] * 5
         for f in ("simint_compute_overlap", "simint_compute_ke", "simint_compute_osoei_overlap",
