@@ -220,7 +220,7 @@ void *simint_hip_stream(void);                /* hipStream_t of the calling thre
 int   simint_hip_set_stream(void * stream);
 /* Lanes per quartet (1, 2, 4, 8 or 16) of the calling thread's later
  * lane-per-quartet simint_hip_compute_eri_list launches (and of the terms of
- * a derivative list): each lane sums a
+ * a derivative list whose HRR transfers two units of AM at most): each lane sums a
  * strided share of the quartet's primitive quartets and the shares are added
  * across the lanes before the HRR.  0 (the default): chosen by list length,
  * so that a launch has about 65536 lanes.  Returns the previous setting or

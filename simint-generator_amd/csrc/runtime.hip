@@ -1609,6 +1609,7 @@ EriListArgs list_args(const simint_hip_pairs *P, const simint_hip_pairs *Q, long
 }
 
 thread_local int t_list_split = 0;   // 0: by list length
+constexpr int kReorderAM = 2;        // the component-lane lists' SHARE_AM (emitter/hip_cpl.py)
 
 // Launcher of a list of n quartets of one class over these pairs.  A list is
 // taken to be of even depth if the pairs' mean depths multiply to half their
@@ -1715,8 +1716,10 @@ long long deriv1_list(const simint_hip_pairs *P, const simint_hip_pairs *Q, long
         a.ostride = t.nc;
         // several lanes a quartet add its primitive quartets in another order,
         // which the HRR and the weight 2a amplify: only where the HRR transfers
-        // one unit of AM at most (six (sd|pp) quartets on a lane each took 1.2 ms)
-        if (std::min(t.am[0], t.am[1]) + std::min(t.am[2], t.am[3]) <= 1) a.split = list_split(nquartet, a.depth);
+        // kReorderAM units of AM at most (six (sd|pp) quartets on a lane each
+        // took 1.2 ms; 1500 derivatives move by 1.1e-14 of their norm with a
+        // limit of 1 or 2, by 1.2e-9 with 3)
+        if (std::min(t.am[0], t.am[1]) + std::min(t.am[2], t.am[3]) <= kReorderAM) a.split = list_split(nquartet, a.depth);
         if ((e = fns[k](&a, c.s)) != hipSuccess) { set_err("class kernel launch", e); return SIMINT_ERROR_HIP; }
         if (t.sign > 0) d.plus[t.centre] = a.out;
         else d.minus[t.centre] = a.out;

@@ -74,18 +74,22 @@ SPLIT_W = 4              # between so many wavefronts (primitive quartets: up to
 # where that shortens the longest wavefront's work to DEEP_GAIN of it.  The
 # paths to the tops are walked by more of them: about 1.3 times the work in
 # all, so longer lists, which fill the chip, do not.  256 classes of 32
-# quartets: 13.4 ms with four wavefronts a group, 12.6 with eight.
+# quartets: 16.0 ms with four wavefronts a group, 15.1 with eight.
 DEEP_GROUPS = 64
 DEEP_GAIN = 0.75
 SUM_VALUES = 8           # accumulators added per round where primitive quartets are shared
-# The most AM transferred in the HRR of a class that shares them.  On the
-# mixed-class stream (300000 quartets in a 30-bohr cube) sharing moved
-# integrals of classes above 3 by up to 8e-6 of the set's root mean square
-# (8e-9 of its norm), of the others by at most 1e-10; but as terms of first
-# derivatives, weighted by 2a, classes of 3 moved 1500 derivatives by up to
-# 2e-8 of their norm, classes of 2 by 3e-11, of 1 by 4e-13 (12 seeds).  What
-# it is worth, with limits of 3, 2 and 1: 8192 quartets 12.8, 16.0 and 20.4
-# ms, 300000 quartets 44.2, 47.8 and 52.9, 1500 derivatives 48, 66 and 83.
+# The most AM transferred in the HRR of a class that shares them: another order
+# of the sum rounds otherwise, and the HRR amplifies it.  On the mixed-class
+# stream (300000 quartets in a 30-bohr cube, 8 seeds) sharing moved a set by up
+# to 2.5e-14 of its norm and single integrals by 1.8e-10 of its root mean
+# square.  As terms of first derivatives, weighted by 2a, classes of 3 moved
+# 1500 derivatives by up to 2e-8 of their norm, classes of 2 by 7e-12 (12
+# seeds).  The lanes that share a derivative list's lane-per-quartet quartet
+# keep the same limit (runtime.hip): with 2 they move it by 1.1e-14, with 3 by
+# 1.2e-9.  Plain lane-per-quartet lists have none (classes of 3: 2.1e-12 of the
+# norm, 2.8e-8 of the root mean square).  What sharing is worth, with limits of
+# 3, 2 and 1: 8192 quartets 12.8, 16.0 and 20.4 ms, 300000 quartets 44.2, 47.8
+# and 52.9, 1500 derivatives 48, 66 and 83; with the lanes at 2 as well 60.
 SHARE_AM = 2
 
 # primitive-quartet block of the local data share, in doubles
