@@ -223,7 +223,8 @@ int   simint_hip_set_stream(void * stream);
  * a derivative list whose HRR transfers two units of AM at most): each lane sums a
  * strided share of the quartet's primitive quartets and the shares are added
  * across the lanes before the HRR.  0 (the default): chosen by list length,
- * so that a launch has about 65536 lanes.  Returns the previous setting or
+ * so that a launch has about 65536 lanes, and by the deepest quartet, which
+ * has no more lanes than about its primitive quartets.  Returns the previous setting or
  * a negative SIMINT_ERROR_*.  No counterpart in the reference (its kernels
  * vectorise over kets on the CPU). */
 int   simint_hip_set_list_split(int lanes);

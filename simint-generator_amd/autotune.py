@@ -263,11 +263,11 @@ def tune_split(a):
 
 
 def tune_even(a):
-    """Lists of 50 to 12800 quartets of one depth: for every class whose list
+    """Lists of 50 to 51200 quartets of one depth: for every class whose list
     kernel (after the family tuning) is component-lane, the number of primitive
     quartets from which the lane-per-quartet kernel is taken, below 16 primitive
-    quartets a quartet (timed at 1, the longest list only) and from there on
-    (timed at 16 and 256; the number that makes the timings' product least)."""
+    quartets a quartet (timed at 1 and 4) and from there on (timed at 16 and
+    256): the number that makes the timings' product least."""
     import itertools
     import math
     import numpy as np
@@ -277,19 +277,21 @@ def tune_even(a):
     L = simint.lib()
     if os.path.exists(a.out):
         simint.apply_tuning(a.out)
-    lens = (50, 200, 800, 3200, 12800)
+    lens = (50, 200, 800, 3200, 12800, 51200)
     rng = np.random.default_rng(0)
     sets = {}
-    for la, lb, depth in itertools.product(range(4), range(4), (1, 2, 4)):
-        shells = [(l, tuple(rng.uniform(0, 4, 3)), list(np.exp(rng.uniform(np.log(0.1), np.log(20), depth))),
-                   list(rng.uniform(0.1, 1.0, depth))) for _ in range(64) for l in (la, lb)]
+    for la, lb, k1, k2 in itertools.product(range(4), range(4), (1, 2, 4), (1, 2, 4)):
+        if k2 > k1:
+            continue
+        shells = [(l, tuple(rng.uniform(0, 4, 3)), list(np.exp(rng.uniform(np.log(0.1), np.log(20), k))),
+                   list(rng.uniform(0.1, 1.0, k))) for _ in range(64) for l, k in ((la, k1), (lb, k2))]
         basis = simint.Basis(shells)
         hp = simint.Pairs.from_pairs(basis, [(2 * k, 2 * k + 1) for k in range(64)])
-        sets[la, lb, depth] = simint.DevicePairs(hp)
+        sets[la, lb, k1 * k2] = simint.DevicePairs(hp)
         hp.free()
         basis.free()
     index = [torch.from_numpy(rng.integers(0, 64, lens[-1]).astype(np.int32)).cuda() for _ in range(2)]
-    out = torch.empty(lens[-1] * 10000, dtype=torch.float64, device="cuda")
+    out = torch.empty(lens[-1] * 3600, dtype=torch.float64, device="cuda")
     stream = torch.cuda.ExternalStream(L.simint_hip_stream())
 
     def ms(P, Q, n):
@@ -311,18 +313,17 @@ def tune_even(a):
         t = {}
         for fam in (1, 7):
             L.simint_hip_set_class_list_kernel(*cls, fam)
-            for depth, n in [(1, lens[-1])] + [(d, n) for d in (2, 4) for n in lens]:
-                t[fam, depth, n] = ms(sets[cls[0], cls[1], depth], sets[cls[2], cls[3], depth], n)
-
-        def cost(line):
-            return sum(math.log(t[1 if n * d ** 4 >= line else 7, d, n]) for d in (2, 4) for n in lens)
-        never = 1 << 40
-        deep = min([never] + sorted({n * d ** 4 for d in (2, 4) for n in lens}, reverse=True), key=cost)
-        shallow = lens[-1] if t[1, 1, lens[-1]] < 0.97 * t[7, 1, lens[-1]] else 0
-        if deep < never or shallow:
-            name = quartets.simint_class_name(cls)
-            even[name] = [shallow, deep if deep < never else 0]
-            print("%-8s %s" % (name, even[name]), flush=True)
+            for kp, kq in ((1, 1), (2, 2), (4, 4), (16, 16)):
+                for n in lens:
+                    t[fam, kp * kq, n] = ms(sets[cls[0], cls[1], kp], sets[cls[2], cls[3], kq], n)
+        line = []
+        for depths in ((1, 4), (16, 256)):
+            def cost(at):
+                return sum(math.log(t[1 if at and n * k >= at else 7, k, n]) for k in depths for n in lens)
+            line.append(min([0] + sorted({n * k for k in depths for n in lens}, reverse=True), key=cost))
+        if any(line):
+            even[quartets.simint_class_name(cls)] = line
+            print("%-8s %s" % (quartets.simint_class_name(cls), line), flush=True)
     L.simint_hip_reset_class_kernels()
     for d in sets.values():
         d.free()

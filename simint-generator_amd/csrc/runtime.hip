@@ -1609,6 +1609,7 @@ EriListArgs list_args(const simint_hip_pairs *P, const simint_hip_pairs *Q, long
 }
 
 thread_local int t_list_split = 0;   // 0: by list length
+constexpr long long kFullList = 65536;   // lanes that fill the card
 constexpr int kReorderAM = 2;        // the component-lane lists' SHARE_AM (emitter/hip_cpl.py)
 
 // Launcher of a list of n quartets of one class over these pairs.  A list is
@@ -1629,14 +1630,15 @@ simint_list_launch_fn list_launch(const simint_hip_pairs *P, const simint_hip_pa
 // that the launch has about 65536 lanes (a short list of one class otherwise
 // occupies a few dozen wavefronts), up to 16; up to a whole wavefront while
 // it has fewer than 16384 (a list of six quartets of up to 1296 primitive
-// quartets otherwise leaves 81 of them to one lane) and a quartet has as many
-// primitive quartets: 50 uncontracted (pp|pp) quartets take 9.7 us with 16
-// lanes each and 11.7 with 64.
+// quartets otherwise leaves 81 of them to one lane).  Never many more than the
+// deepest has primitive quartets, the others of which would wait: uncontracted
+// (pp|pp) quartets take 6.6 us a list of 50 with one lane each, 10.1 with 16
+// and 11.7 with 64, a list of 5000 8.1 and 24.2 (one and 16).
 int list_split(long long n, long long depth)
 {
     if (t_list_split > 0) return t_list_split;
     int s = 1;
-    while (s < 16 && n * s < 65536) s *= 2;
+    while (s < 16 && n * s < kFullList && s < depth) s *= 2;
     while (s < 64 && n * s < 16384 && s < depth) s *= 2;
     return s;
 }
@@ -1687,11 +1689,16 @@ long long deriv1_list(const simint_hip_pairs *P, const simint_hip_pairs *Q, long
     const int am[4] = {P->am1, P->am2, Q->am1, Q->am2};
     const DerivPlan dp = deriv1_plan(am);
     simint_list_launch_fn fns[8];
+    bool lanes[8];
     for (int k = 0; k < dp.nt; k++) {
         const DerivPlan::T &t = dp.t[k];
         fns[k] = nullptr;
+        lanes[k] = std::min(t.am[0], t.am[1]) + std::min(t.am[2], t.am[3]) <= kReorderAM;
         if (t.am[0] <= kTermMaxAM && t.am[1] <= kTermMaxAM && t.am[2] <= kTermMaxAM && t.am[3] <= kTermMaxAM)
-            fns[k] = simint_dispatch_list(t.am[0], t.am[1], t.am[2], t.am[3]);
+            // the lane-per-quartet kernel of even lists where it may have its lanes or needs none
+            fns[k] = lanes[k] || nquartet >= kFullList
+                         ? list_launch(P, Q, t.am[0], t.am[1], t.am[2], t.am[3], nquartet)
+                         : simint_dispatch_list(t.am[0], t.am[1], t.am[2], t.am[3]);
         if (!fns[k]) { t_err = "class not built"; return SIMINT_ERROR_UNSUPPORTED; }
     }
     if (nquartet == 0) return 0;
@@ -1719,7 +1726,7 @@ long long deriv1_list(const simint_hip_pairs *P, const simint_hip_pairs *Q, long
         // kReorderAM units of AM at most (six (sd|pp) quartets on a lane each
         // took 1.2 ms; 1500 derivatives move by 1.1e-14 of their norm with a
         // limit of 1 or 2, by 1.2e-9 with 3)
-        if (std::min(t.am[0], t.am[1]) + std::min(t.am[2], t.am[3]) <= kReorderAM) a.split = list_split(nquartet, a.depth);
+        if (lanes[k]) a.split = list_split(nquartet, a.depth);
         if ((e = fns[k](&a, c.s)) != hipSuccess) { set_err("class kernel launch", e); return SIMINT_ERROR_HIP; }
         if (t.sign > 0) d.plus[t.centre] = a.out;
         else d.minus[t.centre] = a.out;

@@ -24,7 +24,8 @@ def test_one_limit():
     from emitter import hip_cpl
     text = open(os.path.join(PKG, "csrc", "runtime.hip")).read()
     assert int(re.search(r"constexpr int kReorderAM = (\d+);", text)[1]) == hip_cpl.SHARE_AM
-    assert "+ std::min(t.am[2], t.am[3]) <= kReorderAM" in text
+    assert "lanes[k] = std::min(t.am[0], t.am[1]) + std::min(t.am[2], t.am[3]) <= kReorderAM;" in text
+    assert "if (lanes[k]) a.split = list_split(" in text
 
 
 @pytest.mark.gpu
