@@ -10,6 +10,7 @@ pairs of depth 1-3 in an 8-bohr cube), and writes the fastest family per class t
 build to set each class's default):
 
     python simint-generator_amd/autotune.py [--natom 16] [--reps 3] [--out PATH]
+    python simint-generator_amd/autotune.py --lanes     # small launches ("lane_items")
     python simint-generator_amd/autotune.py --list [--split] [--even]   # quartet-list kernels
 
 --list --split also times the lanes per quartet of the lane-per-quartet
@@ -43,7 +44,12 @@ def main():
     ap.add_argument("--even", action="store_true",
                     help="with --list: also time lists of one depth in the classes whose list kernel is "
                          "component-lane (merges 'list_even' into the output file)")
+    ap.add_argument("--lanes", action="store_true",
+                    help="time the component-lane kernels against the lane-per-quartet ones on few items (merges "
+                         "'lane_items' into the output file)")
     a = ap.parse_args()
+    if a.lanes:
+        return tune_lanes(a)
     if a.list:
         tune_lists(a)
         if a.split:
@@ -260,6 +266,73 @@ def tune_split(a):
     with open(a.out, "w") as f:
         json.dump(doc, f, indent=1, sort_keys=True)
     print("wrote", a.out, "(%d classes with a fixed lane count)" % len(split))
+
+
+def tune_lanes(a):
+    """Items (a bra against 64 kets) up to which a launch of a class that runs
+    the lane-per-quartet kernel is not slower in the component-lane one, for
+    1, 4, 9 and 16 and more (16, 36, 256) primitive quartets.  The other
+    kernel, which small launches do not run, is timed on 256 items: up to one
+    for every SIMD it takes the time of one (uncontracted quartets, which mostly
+    store, a little more, so their line comes out high)."""
+    import itertools
+    import numpy as np
+    import torch
+    import quartets
+    import simint
+    from emitter import hip_lpq
+    L = simint.lib()
+    items = (4, 16, 32, 64, 96, 128)
+    rng = np.random.default_rng(0)
+    sets = {}
+    for la, lb, depth in itertools.product(range(4), range(4), (1, 2, 3, 4)):
+        shells = [(l, tuple(rng.uniform(0, 4, 3)), list(np.exp(rng.uniform(np.log(0.1), np.log(20), depth))),
+                   list(rng.uniform(0.1, 1.0, depth))) for _ in range(64) for l in (la, lb)]
+        basis = simint.Basis(shells)
+        hp = simint.Pairs.from_pairs(basis, [(2 * (k % 64), 2 * (k % 64) + 1) for k in range(256)])
+        sets[la, lb, depth] = simint.DevicePairs(hp)
+        hp.free()
+        basis.free()
+    out = torch.empty(256 * 64 * 1296, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+
+    def us(cls, dp, dq, n):
+        nket = np.full(n, 64, dtype=np.int32)
+        off = np.arange(n, dtype=np.int64) * 64 * int(np.prod([simint.ncart(l) for l in cls]))
+        best = 1e30
+        for rep in range(a.reps + 1):
+            t0 = time.perf_counter()
+            for _ in range(10):
+                simint.compute_range(sets[cls[0], cls[1], dp], sets[cls[2], cls[3], dq], 0, None, nket, off,
+                                     out.data_ptr())
+            simint.synchronize()
+            if rep > 0:
+                best = min(best, time.perf_counter() - t0)
+        return best
+    found = {}
+    for cls in itertools.product(range(4), repeat=4):
+        if hip_lpq.share_kind(cls) != "lanes" or L.simint_hip_class_kernel(*cls) != 1:
+            continue
+        most = []
+        for depths in (((1, 1),), ((2, 1),), ((3, 1),), ((2, 2), (3, 2), (4, 4))):
+            good = items
+            for dp, dq in depths:
+                L.simint_hip_set_class_kernel(*cls, 1)
+                ref = us(cls, dp, dq, 256)
+                L.simint_hip_set_class_kernel(*cls, 7)
+                t = [us(cls, dp, dq, n) for n in items]
+                good = [n for k, n in enumerate(items) if n in good and max(t[:k + 1]) <= 1.03 * ref]
+            most.append(max(good, default=0))
+        found[quartets.simint_class_name(cls)] = most
+        print("%-8s %s" % (quartets.simint_class_name(cls), most), flush=True)
+    L.simint_hip_reset_class_kernels()
+    for d in sets.values():
+        d.free()
+    doc = json.load(open(a.out)) if os.path.exists(a.out) else {}
+    doc["lane_items"] = found
+    with open(a.out, "w") as f:
+        json.dump(doc, f, indent=1, sort_keys=True)
+    print("wrote", a.out, "(%d classes)" % len(found))
 
 
 def tune_even(a):

@@ -373,8 +373,8 @@ EVEN_DEPTH = 16
 
 def load_tuning(pkg_root, key="family", names=FAMILIES):
     """Tuned value per class from tuning.json ("family": prefix kernels,
-    "list_family": quartet-list kernels, "deep_family", "list_even"); names
-    maps it to a number (None: as it is)."""
+    "list_family": quartet-list kernels, "deep_family", "list_even",
+    "lane_items"); names maps it to a number (None: as it is)."""
     path = os.path.join(pkg_root, "tuning.json")
     if not os.path.exists(path):
         return {}
@@ -396,9 +396,10 @@ def generate(pkg_root, include_root, maxam, lpq_ok=None):
     lpq = [am for am in cls if lpq_candidate(am)]
     gterms = deriv_term_classes(maxam)
     wpq = list(cls) + gterms
+    lane_items = load_tuning(pkg_root, "lane_items", None)
     for am in lpq:
         _write(os.path.join(gen, "eri_lpq_%s.hip" % hip_lpq.class_name(am)),
-               hip_lpq.emit_lpq(am, mixed=mixed_candidate(am)))
+               hip_lpq.emit_lpq(am, mixed=mixed_candidate(am), lane_items=lane_items.get(am)))
     for am in wpq:
         _write(os.path.join(gen, "eri_wpq_%s.hip" % hip_lpq.class_name(am)), hip_wpq.emit_wpq(am))
     cpl = [am for am in wpq if hip_cpl.candidate(am)]

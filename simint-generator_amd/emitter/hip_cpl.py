@@ -37,14 +37,18 @@ generator/ostei/OSTEI_Writer.cpp:595-702; VRR: OSTEI_VRR_Writer.cpp:95-125;
 HRR: OSTEI_HRR_Writer.cpp:22-99), so the values are theirs bit for bit
 where the contraction runs in one lane there.
 
-Bound: FP64 issue in the tree (three to five operations per value) with the
-local data share close behind; at one or two wavefronts a SIMD its latency
-shows.  Lists of the mixed-class stream (all classes one after another,
-100000 quartets): 560 ms with the cooperative and lane-per-quartet kernels,
-77 ms with these; (ff|ff) 11.8 -> 3.6 ms, (ff|fd) 18.9 -> 2.9 ms, (dd|dd)
-5.3 -> 0.8 ms.  Ranges of a 24-atom molecule: (dd|dp) 2.02 -> 0.96 ms,
-(dp|dp) 1.70 -> 1.23, (dd|dd) 0.59 -> 0.32; random pairs: (ff|ff) 76.6 ->
-29.4 ms, (fd|fd) 30.4 -> 5.6.
+Bound: latency at one or two wavefronts a SIMD.  On the 256-atom system
+(dd|dp) issues vector instructions in 42 % of the cycles (three to five FP64
+operations per value), the local data share works in 41 %, HBM at 27 % of its
+rate.  About two thirds of the kernels also keep some of their values in
+scratch: the register bound (Plan.regs) counts the tree and the accumulators,
+while in the HRR a lane holds a whole column.  Lists of the mixed-class stream
+(all classes one after another, 100000 quartets): 560 ms with the cooperative
+and lane-per-quartet kernels; the 186 classes that run these take 94 ms,
+(ff|ff) 11.8 -> 3.4 ms, (ff|fd) 18.9 -> 2.7 ms, (dd|dd) 5.3 -> 0.9 ms.  Ranges
+of a 24-atom molecule: (dd|dp) 2.02 -> 0.96 ms, (dp|dp) 1.70 -> 1.23, (dd|dd)
+0.59 -> 0.32; random pairs: (ff|ff) 76.6 -> 29.4 ms, (fd|fd) 30.4 -> 5.6.
+Screened primitive quartets are left out where a group's quartets all are.
 """
 from functools import lru_cache
 

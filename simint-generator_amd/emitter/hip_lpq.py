@@ -364,7 +364,7 @@ def _emit_fast_setup(w, Ltot):
     w("")
 
 
-def emit_lpq(am, mixed=False):
+def emit_lpq(am, mixed=False, lane_items=None):
     """Source of one class: the prefix kernel, the quartet-list kernel and,
     with mixed=True, the FP32-VRR prefix kernel (eri_lpqm_<class>)."""
     w = _Writer()
@@ -383,12 +383,12 @@ def emit_lpq(am, mixed=False):
     for fp in (("double", "float") if mixed else ("double",)):
         if share_kind(am) in ("sum", "turn"):
             _emit_lpq_prefix(am, w, fp, shared=share_kind(am))
-        _emit_lpq_launcher(am, w, fp)
+        _emit_lpq_launcher(am, w, fp, lane_items)
     return w.text()
 
 
 # Small launches: several wavefronts share an item's primitive quartets, eight
-# at most and no more than it has.  A 12-atom molecule's (ss|ss) launches are a
+# at most and about as many as it has.  A 12-atom molecule's (ss|ss) launches are a
 # few dozen items of up to 1296 primitive quartets: 82 us each with one
 # wavefront an item, 24 us so.
 # Classes without HRR add the wavefronts' sums at the end, while the launch has
@@ -405,17 +405,18 @@ def emit_lpq(am, mixed=False):
 #    wavefront and 84 with four, 1024 of them 140 and 317; two wavefronts are
 #    slower than one always;
 #  * the rest run the component-lane kernel, which spreads a quartet over lanes
-#    instead and gives the same values, up to LANE_ITEMS items and
-#    LANE_ITEMS_PER_DEPTH for each primitive quartet of the deepest: over the
-#    60 classes it takes 0.58, 0.70 and 0.86 of the time with 32, 64 and 128
-#    items of 16 primitive quartets, 0.76, 0.85 and 0.98 with 4, but 1.12, 1.21
-#    and 1.33 with 1.  Where the wide side has AM 2 in all a quartet is 10
-#    lanes' work and LANE_ITEMS_2 the line ((ps|pp): 0.97 with 32, 1.19 with 128).
+#    instead and gives the same values, up to a number of items by class and
+#    depth (LANE_DEPTHS) that tuning.json's "lane_items" holds (autotune.py
+#    --lanes: the most at which it is not slower): over the 60 classes it takes
+#    0.58, 0.70 and 0.86 of the time with 32, 64 and 128 items of 16 primitive
+#    quartets, 0.76, 0.85 and 0.98 with 4, but 1.12, 1.21 and 1.33 with 1; 128
+#    items of 16 0.42 of it for (dd|ds) and 1.19 for (ps|pp).  Classes it does
+#    not name: LANE_ITEMS_PER_DEPTH for each primitive quartet, up to LANE_ITEMS.
 SHARE_ITEMS = 2048
 SHARE_TOPS = 36
 LANE_ITEMS = 128
-LANE_ITEMS_2 = 32
 LANE_ITEMS_PER_DEPTH = 8
+LANE_DEPTHS = (4, 9, 16)    # "lane_items": below 4 primitive quartets, 9, 16, and from there on
 SHARE_SUM = 8       # contracted values added per round at the end (classes without HRR)
 
 
@@ -441,7 +442,7 @@ def share_waves(am):
     return 8 if ntop <= 16 else 4 if ntop <= 32 else 2
 
 
-def _emit_lpq_launcher(am, w, fp):
+def _emit_lpq_launcher(am, w, fp, lane_items=None):
     kname = ("lpqm_%s" if fp == "float" else "lpq_%s") % class_name(am)
     kind, most = share_kind(am), share_waves(am)
     if kind == "lanes" and fp == "double":
@@ -452,15 +453,19 @@ def _emit_lpq_launcher(am, w, fp):
     if kind:
         w("    const long long depth = a->depth > 0 ? a->depth : 4096;   // unknown: as deep ones")
     if kind == "lanes":
-        g = graph(*am)
-        most_items = LANE_ITEMS_2 if max(g.e_hi, g.f_hi) == 2 else LANE_ITEMS
-        w("    if (a->nitems <= (%d * depth < %d ? %d * depth : %d)) return simint_launch_cpl_%s(a, s);"
-          % (LANE_ITEMS_PER_DEPTH, most_items, LANE_ITEMS_PER_DEPTH, most_items, class_name(am)))
+        if lane_items:
+            test = "depth < %d ? %d : depth < %d ? %d : depth < %d ? %d : %d" % (
+                LANE_DEPTHS[0], lane_items[0], LANE_DEPTHS[1], lane_items[1], LANE_DEPTHS[2], lane_items[2],
+                lane_items[3])
+        else:
+            test = "%d * depth < %d ? %d * depth : %d" % (LANE_ITEMS_PER_DEPTH, LANE_ITEMS, LANE_ITEMS_PER_DEPTH,
+                                                          LANE_ITEMS)
+        w("    if (a->nitems <= (%s)) return simint_launch_cpl_%s(a, s);" % (test, class_name(am)))
     elif kind == "sum":
         w("    int waves = 1;")
         room = ("a->nitems * waves < %d" % SHARE_ITEMS if len(graph(*am).top_keys) <= SHARE_TOPS
                 else "2 * a->nitems * waves <= %d" % (SHARE_ITEMS // 2))
-        w("    while (waves < %d && 2 * waves <= depth && %s) waves *= 2;" % (most, room))
+        w("    while (waves < %d && waves < depth && %s) waves *= 2;" % (most, room))
         w("    if (waves > 1) {")
         w("        hipLaunchKernelGGL(eri_%s, dim3((unsigned)a->nitems), dim3(64, waves), 0, s, *a);"
           % kname.replace("_", "k_", 1))
@@ -470,8 +475,8 @@ def _emit_lpq_launcher(am, w, fp):
         terms = 2 * 512 * len(graph(*am).top_keys)   # of one wavefront, both buffers
         for waves in (8, 4):
             if waves <= most:
-                w("    if (a->nitems <= %d && depth >= %d%s) {"
-                  % (256 * (160 * 1024 // (waves * terms)), waves, "" if waves == most else " && depth < %d" % most))
+                w("    if (a->nitems <= %d && depth > %d%s) {"
+                  % (256 * (160 * 1024 // (waves * terms)), waves // 2, "" if waves == most else " && depth <= %d" % waves))
                 w("        hipLaunchKernelGGL(eri_%s, dim3((unsigned)a->nitems), dim3(64, %d), %du, s, *a);"
                   % (kname.replace("_", "k_", 1), waves, waves * terms))
                 w("        return hipGetLastError();")
